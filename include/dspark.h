@@ -148,6 +148,20 @@ int dspark_qmm_dequantize(const uint32_t* w, const void* scales, const void* bia
                           dspark_stream stream);
 
 /*
+ * The same product for many rows (prefill widths): y = x . dequant(w)^T for reference-layout w
+ * and bf16 scales / biases, any M >= 1, N >= 1, K % 64 == 0. fp32 accumulation over exact
+ * products, weights never rounded; outputs that are not finite are recomputed as the plain fp32
+ * dequantized product. `bias` (nullable, bf16 [N]) is added to the bf16 product, rounded again.
+ * x 16-byte aligned with ldx % 8 == 0, w 16-byte aligned. Workspace 256-byte aligned, any
+ * contents. Takes the place of the dequantize-then-GEMM of the reference's wide path
+ * (wide_gemm.py:173-232).
+ */
+size_t dspark_qmm_wide_workspace(int64_t M, int64_t K, int64_t N, int bits, int group_size);
+int dspark_qmm_wide(const void* x, int64_t ldx, int64_t M, int64_t K, const uint32_t* w, const void* scales,
+                    const void* biases, int64_t N, int bits, int group_size, const void* bias, void* y, int64_t ldy,
+                    void* workspace, size_t workspace_bytes, dspark_stream stream);
+
+/*
  * Streaming-read bandwidth probe: reads `bytes` (a positive multiple of 16, 16-byte aligned) once
  * with 16-byte non-temporal loads; sink[0] is written only in the (practically impossible) case
  * that the XOR of all words equals a sentinel. Timed by the caller, it gives the measured HBM

@@ -4,9 +4,10 @@
 path's projections are instances of it, and ``small_m_qmm.small_m_matmul`` re-routes their
 calls class-wide (small_m_qmm.py:71-106). Its own ``forward`` is the *stock* path — the
 counterpart of ``mx.quantized_matmul`` that the reference falls through to outside the kernel
-window (small_m_qmm.py:53): dequantize to fp32 and multiply, output in x's dtype. The stock
-path serves shapes and dtypes the kernels do not (prefill widths, fp32 activations); the
-verify window runs on the HIP kernel through the scope.
+window (small_m_qmm.py:53): the product with the weight unrounded and fp32 sums, output in x's
+dtype. bf16 calls of more than 16 rows (prefill widths) run it on the matrix cores
+(``ops.quantized_matmul_wide``); the rest dequantize to fp32 and multiply with torch. The verify
+window runs on its HIP kernels through the scope.
 
 ``QuantizedSwitchLinear`` holds one such matrix per expert (stacked on a leading axis), the
 layout of mlx-lm's ``QuantizedSwitchLinear`` that ``SwitchGLU`` gathers from.
@@ -17,7 +18,7 @@ from __future__ import annotations
 import torch
 from torch import nn
 
-from . import quant
+from . import ops, quant
 
 GROUP = quant.GROUP
 
@@ -70,8 +71,29 @@ class QuantizedLinear(nn.Module):
             bb = (torch.randn(out_features, device=device, generator=generator) * 0.02).to(torch.bfloat16)
         return cls(w, s, b, bb, bits=bits)
 
+    def wide_kernel(self, x: torch.Tensor) -> bool:
+        """Whether the matrix-core kernel (``ops.quantized_matmul_wide``) computes this call: bf16
+        rows and parameters on the GPU, more rows than a verify block (16: up to there the stock
+        product is what the verify kernels are raced against), nothing recording gradients.
+        Every other call keeps the torch product."""
+        w, s, b, bias = self.weight, self.scales, self.biases, self.bias
+        if not x.is_cuda or x.dtype != torch.bfloat16 or b is None or self.mode != "affine":
+            return False
+        if self.bits not in (4, 8) or self.group_size != GROUP or x.dim() < 1:
+            return False
+        k, n = self.in_features, self.out_features
+        params = (w, s, b) if bias is None else (w, s, b, bias)
+        return (x.shape[-1] == k and 16 * k < x.numel() <= k << 24 and 0 < k <= 1 << 22 and 0 < n <= 1 << 24
+                and k % GROUP == 0 and tuple(s.shape) == (n, k // GROUP) and b.shape == s.shape
+                and all(p.dtype == torch.bfloat16 for p in params[1:])
+                and (bias is None or tuple(bias.shape) == (n,))
+                and w.is_contiguous() and w.data_ptr() % 16 == 0 and ops.eager_inference(x, *params))
+
     def stock(self, x: torch.Tensor) -> torch.Tensor:
-        """The stock path: fp32 dequantize + matmul, result in x's dtype."""
+        """The stock path, result in x's dtype: the matrix-core product over exact bf16 fields
+        where :meth:`wide_kernel` takes the call, else fp32 dequantize + matmul."""
+        if self.wide_kernel(x):
+            return ops.quantized_matmul_wide(x, self.weight, self.scales, self.biases, bits=self.bits, bias=self.bias)
         w = quant.dequantize(self.weight, self.scales, self.biases, self.group_size, self.bits)
         y = (x.reshape(-1, x.shape[-1]).to(torch.float32) @ w.t()).to(x.dtype)
         y = y.reshape(*x.shape[:-1], y.shape[-1])

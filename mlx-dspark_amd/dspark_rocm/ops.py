@@ -133,6 +133,54 @@ def quantized_matmul_multi(x_list, w_list, s_list, b_list, *, group_size: int = 
     return results
 
 
+def eager_inference(*ts: torch.Tensor) -> bool:
+    """Whether a call on these tensors may go straight to a kernel that autograd, tracing, tensor
+    subclasses and function transforms do not see: plain tensors on one ROCm device, nothing that
+    records gradients or tangents, no dispatch or function mode and no transform active."""
+    first = ts[0]
+    if not first.is_cuda or torch.jit.is_tracing() or torch.compiler.is_compiling():
+        return False
+    if torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack():
+        return False
+    if torch._C._functorch.peek_interpreter_stack() is not None:
+        return False
+    if torch.autograd.forward_ad._current_level >= 0:
+        return False
+    grad = torch.is_grad_enabled()
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.device == first.device
+               and t.layout == torch.strided and not (grad and t.requires_grad)
+               and not (t.is_neg() or t._is_zerotensor()) for t in ts)
+
+
+def quantized_matmul_wide(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor, *, bits: int,
+                          group_size: int = GROUP, bias: torch.Tensor | None = None) -> torch.Tensor:
+    """``x [.., K] @ dequant(w)^T (+ bias)`` for many rows (prefill widths) on the matrix cores:
+    exact bf16 products, fp32 sums, weights never rounded (``dspark_qmm_wide``). ``bias`` (bf16
+    [N]) is added to the bf16 product, as a module adds it."""
+    _require_cuda(x, w, scales, biases, bias)
+    for name, t in (("x", x), ("scales", scales), ("biases", biases)) + ((("bias", bias),) if bias is not None else ()):
+        _require_bf16(name, t)
+    _require_packed(w)
+    k, n = int(x.shape[-1]), int(w.shape[0])
+    if w.dim() != 2 or w.shape[1] * 32 != k * bits or tuple(scales.shape) != (n, k // group_size) \
+            or biases.shape != scales.shape or (bias is not None and tuple(bias.shape) != (n,)):
+        raise ValueError(f"x K={k}, weight {tuple(w.shape)}, scales {tuple(scales.shape)}, biases {tuple(biases.shape)}")
+    x2 = x.reshape(-1, k)
+    if x2.stride(-1) != 1 or x2.stride(0) % 8 or not k <= x2.stride(0) <= 1 << 22 or x2.data_ptr() % 16:
+        x2 = x2.clone(memory_format=torch.contiguous_format)
+    w, scales, biases = w.contiguous(), scales.contiguous(), biases.contiguous()
+    bias = None if bias is None else bias.contiguous()
+    m = x2.shape[0]
+    y = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
+    if m and n:
+        with torch.cuda.device(x.device):
+            nbytes = int(_lib.load().dspark_qmm_wide_workspace(m, k, n, bits, group_size))
+            ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=x.device)
+            _lib.call("dspark_qmm_wide", _ptr(x2), x2.stride(0), m, k, _ptr(w), _ptr(scales), _ptr(biases), n, bits,
+                      group_size, _ptr(bias), _ptr(y), y.stride(0), _ptr(ws), nbytes, _stream(x))
+    return y.reshape(*x.shape[:-1], n)
+
+
 class PackedQmm:
     """A quantized [N, K] matrix in the MI355X packed form (``dspark_qmm_pack``): 16-row weight
     tiles in the MFMA lane order plus 16-row x 8-group scale/bias tiles, in one uint8 buffer.

@@ -6,9 +6,12 @@ the product of the leading dims, so a ``[1, L, K]`` prefill counts L) whose shap
 verified allowlist takes the wide path, and the result is **bit-identical** to the stock path
 for that shape; everything else runs the forward installed on entry, unchanged.
 
-What the wide path replaces here. The stock path (:meth:`QuantizedLinear.stock`) dequantizes
-with torch elementwise ops -- unpack through int64, convert, multiply, add: several passes over
-an ``N x K`` fp32 tensor -- and then runs one fp32 GEMM. The wide path produces the same fp32
+What the wide path replaces here. bf16 calls of more than 16 rows never see it: there the stock
+path is already the matrix-core product over the packed weight (:meth:`QuantizedLinear.wide_kernel`),
+and :func:`wide_rows` makes the same call, so the bits agree. For the other activation and scale
+dtypes the stock path dequantizes with torch elementwise ops -- unpack through int64, convert,
+multiply, add: several passes over an ``N x K`` fp32 tensor -- and then runs one fp32 GEMM. The
+wide path produces the same fp32
 weight in one pass (``dspark_qmm_dequantize``: ``(scale * q) + bias``, each operation rounded
 as torch rounds it, no fma contraction) and hands it to the same GEMM call with the same
 operands, so the bits agree by construction; :func:`verified_shapes` still checks every shape
@@ -70,8 +73,11 @@ def shape_key(mod) -> str:
 
 
 def wide_rows(mod, x: torch.Tensor, exact: bool = True) -> torch.Tensor:
-    """The wide path's result for ``mod(x)`` (no routing decision): one dequantize launch,
-    then the GEMM, then the module's bias, in the stock path's order of operations."""
+    """The wide path's result for ``mod(x)`` (no routing decision): the matrix-core product where
+    the stock path takes it, else one dequantize launch, then the GEMM, then the module's bias, in
+    the stock path's order of operations."""
+    if exact and mod.wide_kernel(x):
+        return ops.quantized_matmul_wide(x, mod.weight, mod.scales, mod.biases, bits=int(mod.bits), bias=mod.bias)
     k = x.shape[-1]
     x2 = x.reshape(-1, k)
     if exact or x.dtype == torch.float32:
