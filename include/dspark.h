@@ -331,6 +331,22 @@ int dspark_verify_attention_typed(int dtype, const void* q, int64_t B, int64_t H
                                   dspark_stream stream);
 
 /*
+ * Attention over many query rows (prefill widths): out = softmax(scale * q . k^T) . v, causal (row
+ * i sees keys 0 .. L - M + i) or over all L keys. fp32 scores, softmax and sums; the probabilities
+ * keep their fp32 precision into the second product. q [B, Hq, M, D], K/V [B, Hk, L, D] of dtype
+ * DSPARK_DTYPE_BF16 or _F16 through element strides {batch, head, position} (each a multiple of
+ * 8, positions at most 2^22 elements apart; the last dim contiguous; all 16-byte aligned), D in {64, 128,
+ * 256}, out a contiguous [B, Hq, M, D]. scale > 0; causal needs L >= M. Workspace 16-byte aligned,
+ * any contents. The reference's prefill runs mx.fast.scaled_dot_product_attention here
+ * (multirow_attn.py:50 captures it).
+ */
+size_t dspark_prefill_attention_workspace(int64_t B, int64_t Hq, int64_t Hk, int64_t M, int64_t L, int64_t D);
+int dspark_prefill_attention(int dtype, const void* q, const int64_t q_strides[3], int64_t B, int64_t Hq, int64_t M,
+                             int64_t D, const void* k, const void* v, const int64_t k_strides[3],
+                             const int64_t v_strides[3], int64_t Hk, int64_t L, float scale, int causal, void* out,
+                             void* workspace, size_t workspace_bytes, dspark_stream stream);
+
+/*
  * Verify attention over a quantized KV cache: the state of mlx-lm's QuantizedKVCache, which
  * the reference's targets build when kv_bits is set (target.py:166-184; its shape is read back
  * at calibrate.py:225-238). K and V are each

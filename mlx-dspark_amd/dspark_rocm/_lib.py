@@ -92,6 +92,10 @@ SIGNATURES: dict[str, tuple] = {
     "dspark_qmm_wide_workspace": (c_size_t, [c_i64, c_i64, c_i64, c_int, c_int]),
     "dspark_qmm_wide": (c_int, [c_void_p, c_i64, c_i64, c_i64, c_void_p, c_void_p, c_void_p, c_i64, c_int, c_int,
                                 c_void_p, c_void_p, c_i64, c_void_p, c_size_t, c_void_p]),
+    "dspark_prefill_attention_workspace": (c_size_t, [c_i64] * 6),
+    "dspark_prefill_attention": (c_int, [c_int, c_void_p, c_i64_p, c_i64, c_i64, c_i64, c_i64, c_void_p, c_void_p,
+                                         c_i64_p, c_i64_p, c_i64, c_i64, c_float, c_int, c_void_p, c_void_p,
+                                         c_size_t, c_void_p]),
     "dspark_qmm_affine_noalloc": (c_int, [c_void_p, c_i64, c_i64, c_i64, c_void_p, c_void_p, c_void_p, c_i64,
                                           c_int, c_int, c_void_p, c_i64, c_void_p]),
     "dspark_qmm_noalloc_reset": (c_int, [c_void_p]),

@@ -4,8 +4,9 @@ the reference; multirow_attn.py:50 and sdpa_split.py:38 capture and replace it).
 
 Callers look the function up on this module at call time (``fast.scaled_dot_product_attention``)
 so the scopes in :mod:`.sdpa_split` and :mod:`.multirow_attn` can route it. The function
-defined here is the stock path: fp32 scores and softmax, output in q's dtype, computed with
-torch ops on q's device.
+defined here is the stock path: fp32 scores and softmax, output in q's dtype. bf16 and fp16 calls
+of more than 16 rows run it on the matrix cores (``ops.prefill_attention``), the rest with torch
+ops on q's device.
 
 Semantics (MLX's): q [B, Hq, qL, D], k/v [B, Hk, L, D] with Hq % Hk == 0 (GQA: query head h
 reads KV head h // (Hq/Hk)). ``mask`` is None, the string "causal" (row i sees keys
@@ -17,6 +18,10 @@ every row's softmax normaliser without a value.
 from __future__ import annotations
 
 import torch
+
+from . import ops
+
+PREFILL_MIN_ROWS = 17   # up to a verify block (16 rows) the torch ops are what its kernels are raced against
 
 
 def _expand_kv(t: torch.Tensor, hq: int) -> torch.Tensor:
@@ -33,11 +38,37 @@ def causal_mask(q_len: int, kv_len: int, device=None) -> torch.Tensor:
     return j <= (kv_len - q_len + i)
 
 
+def prefill_kernel(q, k, v, scale, mask, sinks) -> bool:
+    """Whether ``ops.prefill_attention`` computes this call: bf16 or fp16 rows on the GPU, more of
+    them than a verify block, no mask but "causal", the kernel's head dims and strides, nothing
+    recording gradients. Every other call keeps the torch ops."""
+    if sinks is not None or not (mask is None or (isinstance(mask, str) and mask == "causal")):
+        return False
+    if not isinstance(q, torch.Tensor) or not q.is_cuda or q.dim() != 4 or k.dim() != 4 or k.shape != v.shape:
+        return False
+    B, Hq, qL, D = q.shape
+    Hk, L = k.shape[1], k.shape[2]
+    if q.dtype not in ops.ATTN_DTYPES or k.dtype != q.dtype or v.dtype != q.dtype or D not in ops.QUANT_HEAD_DIMS:
+        return False
+    if k.shape[0] != B or k.shape[3] != D or not Hk or Hq % Hk or not B or not PREFILL_MIN_ROWS <= qL <= 1 << 22:
+        return False
+    if not (1 <= L <= 1 << 28 and max(B, Hq) <= 65535 and B * Hq * qL <= 1 << 28) or (mask is not None and L < qL):
+        return False
+    if not isinstance(scale, (int, float)) or not 1e-30 < scale < 1e30:
+        return False
+    for t in (q, k, v):
+        if t.stride(3) != 1 or t.data_ptr() % 16 or t.stride(2) > 1 << 22 or any(t.stride(i) % 8 for i in range(3)):
+            return False
+    return ops.eager_inference(q, k, v)
+
+
 def _stock_sdpa(q, k, v, *, scale, mask=None, sinks=None):
     B, Hq, qL, D = q.shape
     L = k.shape[2]
     if k.shape[1] == 0 or Hq % k.shape[1]:
         raise ValueError(f"Hq={Hq} is not a multiple of Hk={k.shape[1]}")
+    if prefill_kernel(q, k, v, scale, mask, sinks):
+        return ops.prefill_attention(q, k, v, scale=scale, causal=mask is not None)
     kk = _expand_kv(k, Hq).to(torch.float32)
     vv = _expand_kv(v, Hq).to(torch.float32)
     s = torch.matmul(q.to(torch.float32), kk.transpose(-1, -2).contiguous()) * float(scale)

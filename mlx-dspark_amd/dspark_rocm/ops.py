@@ -536,6 +536,26 @@ def _launch_attention(dt, q, k, v, out, out_strides, scale, causal, tree_anc, ws
     return out
 
 
+def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, scale: float,
+                      causal: bool = True) -> torch.Tensor:
+    """Attention over many query rows on the matrix cores (``dspark_prefill_attention``): q
+    [B, Hq, M, D], k/v [B, Hk, L, D], bf16 or fp16, D in ``QUANT_HEAD_DIMS``, any batch / head /
+    position strides (multiples of 8 elements, 16-byte aligned rows). fp32 scores, probabilities
+    and sums; causal from the bottom right (needs L >= M). Returns a contiguous [B, Hq, M, D]."""
+    _require_cuda(q, k, v)
+    dt = _attn_dtype(q, k, v)
+    _attn_shapes(q, k, v)
+    B, Hq, M, D = q.shape
+    Hk, L = k.shape[1], k.shape[2]
+    out = torch.empty((B, Hq, M, D), dtype=q.dtype, device=q.device)
+    with torch.cuda.device(q.device):
+        nbytes = int(_lib.load().dspark_prefill_attention_workspace(B, Hq, Hk, M, L, D))
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
+        _lib.call("dspark_prefill_attention", dt, _ptr(q), _i64x3(q), B, Hq, M, D, _ptr(k), _ptr(v), _i64x3(k),
+                  _i64x3(v), Hk, L, float(scale), int(bool(causal)), _ptr(out), _ptr(ws), nbytes, _stream(q))
+    return out
+
+
 def verify_attention_blocks(B: int, Hq: int, Hk: int, mq: int, D: int, L: int) -> int:
     return int(_lib.load().dspark_verify_attention_blocks(B, Hq, Hk, mq, D, L))
 

@@ -1,0 +1,144 @@
+"""GPU: attention over many query rows (``dspark_prefill_attention``) behind the stock entry point.
+
+Against float64 attention of the same inputs. Bound per output: half a unit of the output type, plus
+the errors of the fp32 path: a score is off by at most (D + 2) units of 2^-24 of scale * sum |q k|
+and its exponent's argument by as much again of its size, a probability by that and the unit 2^-22 of
+its pieces, the two sums over L keys by L / 16 units (16 keys a lane are added in turn, 16 or more in
+the matrix core); numerator and denominator both, over sum p |v|.
+Sizes sit at the edges of the 32-row waves, 128-row workgroups, 32 / 64-key tiles and key splits.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+UNIT = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+
+
+def _inputs(dev, b, hq, hk, m, L, d, dtype, seed=0, qscale=2.0):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    mk = lambda h, n, s: (torch.randn((b, h, n, d), generator=g, device=dev) * s).to(dtype)  # noqa: E731
+    return mk(hq, m, qscale), mk(hk, L, 1.0), mk(hk, L, 1.0)
+
+
+def _reference(q, k, v, scale, causal):
+    """(float64 attention, sum p |v|, largest scale * sum |q k| of a row)"""
+    hq, m, L = q.shape[1], q.shape[2], k.shape[2]
+    rep = hq // k.shape[1]
+    kk, vv = (t.double().repeat_interleave(rep, dim=1) for t in (k, v))
+    kt = kk.transpose(-1, -2).contiguous()
+    s = torch.matmul(q.double(), kt) * scale
+    mag = torch.matmul(q.double().abs(), kt.abs()) * scale
+    if causal:
+        i, j = torch.arange(m, device=q.device)[:, None], torch.arange(L, device=q.device)[None]
+        s = s.masked_fill(j > L - m + i, float("-inf"))
+    p = torch.softmax(s, -1)
+    return torch.matmul(p, vv), torch.matmul(p, vv.abs()), mag.amax(-1, keepdim=True)
+
+
+def _check(out, q, k, v, scale, causal, what=""):
+    ref, pv, mag = _reference(q, k, v, scale, causal)
+    amp = 2 * (2 * (q.shape[-1] + 2) * mag + 8 + k.shape[2] / 16) * 2.0 ** -24
+    bound = UNIT[q.dtype] * (ref.abs() + amp * pv) + amp * pv + 2.0 ** -25
+    worst = float(((out.double() - ref).abs() - bound).max())
+    assert out.shape == ref.shape and out.dtype == q.dtype and out.is_contiguous()
+    assert worst <= 0, f"{what}: error exceeds its bound by {worst}"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("b,hq,hk,m,L", [(1, 1, 1, 17, 17), (1, 4, 1, 32, 33), (2, 6, 2, 43, 64), (1, 8, 8, 129, 129),
+                                         (1, 8, 2, 33, 1500), (1, 5, 1, 100, 257), (1, 16, 1, 24, 31 + 24),
+                                         (1, 32, 8, 300, 1301), (1, 64, 8, 65, 2048)])
+def test_matches_float64_attention(dev, b, hq, hk, m, L, d, dtype):
+    from dspark_rocm import fast
+
+    q, k, v = _inputs(dev, b, hq, hk, m, L, d, dtype)
+    for mask in ("causal", None):
+        assert fast.prefill_kernel(q, k, v, d ** -0.5, mask, None)
+        out = fast.scaled_dot_product_attention(q, k, v, scale=d ** -0.5, mask=mask)
+        _check(out, q, k, v, d ** -0.5, mask == "causal", f"{b}x{hq}/{hk}x{m}x{L}x{d} {mask}")
+
+
+def test_views_of_a_cache_and_of_projections(dev):
+    """A cache's filled rows and [B, L, H, D] projections seen as [B, H, L, D] are read in place, to
+    the bits of their contiguous copies."""
+    from dspark_rocm import fast
+
+    q, k, v = _inputs(dev, 2, 8, 2, 70, 190, 128, torch.bfloat16)
+    want = fast.scaled_dot_product_attention(q, k, v, scale=0.1, mask="causal")
+    _check(want, q, k, v, 0.1, True)
+    big = torch.full((2, 2, 256, 128), float("nan"), dtype=k.dtype, device=dev)
+    kc, vc = big.clone(), big.clone()
+    kc[:, :, :190], vc[:, :, :190] = k, v
+    qt = q.transpose(1, 2).contiguous().transpose(1, 2)
+    kt = k.transpose(1, 2).contiguous().transpose(1, 2)
+    for qq, kk, vv in ((q, kc[:, :, :190], vc[:, :, :190]), (qt, kt, v)):
+        assert fast.prefill_kernel(qq, kk, vv, 0.1, "causal", None)
+        got = fast.scaled_dot_product_attention(qq, kk, vv, scale=0.1, mask="causal")
+        assert torch.equal(got, want)
+
+
+def test_calls_that_keep_the_torch_ops(dev):
+    from dspark_rocm import fast
+
+    q, k, v = _inputs(dev, 1, 4, 2, 20, 40, 64, torch.bfloat16)
+    ok = lambda q=q, k=k, v=v, scale=0.1, mask="causal", sinks=None: fast.prefill_kernel(  # noqa: E731
+        q, k, v, scale, mask, sinks)
+    assert ok()
+    assert not ok(q=q[:, :, :16])
+    assert not ok(q=q.float()) and not ok(q=q.half())
+    assert not ok(mask=torch.ones(20, 40, dtype=torch.bool, device=dev))
+    assert not ok(sinks=torch.zeros(4, device=dev))
+    assert not ok(k=k[:, :, :19], v=v[:, :, :19]) and ok(k=k[:, :, :19], v=v[:, :, :19], mask=None)
+    assert not ok(scale=0.0) and not ok(scale=-1.0) and not ok(scale=float("inf"))
+    assert not ok(q=q[..., :40], k=k[..., :40], v=v[..., :40])
+    assert not ok(k=k[:, :, :, ::1].transpose(2, 3).contiguous().transpose(2, 3))
+    shifted = torch.zeros(q.numel() + 1, dtype=q.dtype, device=dev)[1:].view(q.shape)
+    assert not ok(q=shifted)
+    qg = q.clone().requires_grad_()
+    assert not ok(q=qg)
+    fast.scaled_dot_product_attention(qg, k, v, scale=0.1, mask="causal").float().sum().backward()
+    assert qg.grad is not None and bool(torch.isfinite(qg.grad).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_large_scores_and_non_finite_values(dev, dtype):
+    """Scores of any size keep the softmax exact at its maximum; a row whose scores hold an infinity
+    or a NaN is NaN, as the torch ops have it, and the other rows are what they were."""
+    from dspark_rocm import fast
+
+    q, k, v = _inputs(dev, 1, 2, 1, 40, 700, 64, dtype)
+    big = (q.float() * 200).to(dtype), (k.float() * 200).to(dtype)
+    ref, _, _ = _reference(*big, v, 50.0, True)
+    out = fast.scaled_dot_product_attention(*big, v, scale=50.0, mask="causal")
+    assert float((out.double() - ref).abs().max()) <= UNIT[dtype] * float(ref.abs().max())
+    want = fast.scaled_dot_product_attention(q, k, v, scale=0.125, mask="causal")
+    q2 = q.clone()
+    q2[0, 1, 7, 3] = float("inf")
+    q2[0, 0, 9, 5] = float("nan")
+    out = fast.scaled_dot_product_attention(q2, k, v, scale=0.125, mask="causal")
+    hit = torch.zeros((2, 40), dtype=torch.bool, device=dev)
+    hit[1, 7] = hit[0, 9] = True
+    assert bool(torch.isnan(out[0][hit]).all()) and torch.equal(out[0][~hit], want[0][~hit])
+
+
+def test_capture_replays_on_new_inputs(dev):
+    from dspark_rocm import fast
+
+    q, k, v = _inputs(dev, 1, 8, 2, 64, 900, 128, torch.bfloat16)   # splits the keys
+    run = lambda: fast.scaled_dot_product_attention(q, k, v, scale=0.1, mask="causal")  # noqa: E731
+    run()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = run()
+    for seed in (1, 2, 3):
+        for t, n in zip((q, k, v), _inputs(dev, 1, 8, 2, 64, 900, 128, torch.bfloat16, seed=seed)):
+            t.copy_(n)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, run())
