@@ -16,16 +16,22 @@
 // (counting sort, stable in pair id). The grouped qmm launches one workgroup per
 // (expert, 16-feature tile); workgroups of unselected experts exit at once, every selected
 // expert's weight tile is streamed once for all of its tokens (<= 16 at verify widths).
+#include <algorithm>
 #include <initializer_list>
 
 #include "dspark_moe_cu.h"
 #include "dspark_moe_rc.h"
 #include "dspark_moe_sk.h"
+#include "dspark_moe_wide.h"
 
 namespace dspark {
 namespace {
 
 constexpr int kRouteThreads = 1024;  // one wave per token, 16 tokens at a time
+// Tokens up to which one workgroup routes them all (a round of 16 takes about 3 us; the second
+// launch of the other way costs as much). 500 tokens: 98 us in one workgroup, 4.7 + 9.8 us in two
+// launches.
+constexpr int kRouteOneGroup = 32;
 
 struct RouteArgs {
   const u16* logits;
@@ -36,6 +42,8 @@ struct RouteArgs {
   int* pos;
   int* ctr;   // nullable: arrival counters of the grouped qmm, cleared here
   int nctr;
+  wide::MoeTile* tiles;  // nullable: the buckets' row tiles, filled to max_tiles entries
+  int tile_rows, max_tiles;
   int M, E, k, renorm;
 };
 
@@ -66,76 +74,65 @@ __device__ __forceinline__ u32 wave_max_u32(u32 v) {
   return max(max(r0, r1), max(r2, r3));
 }
 
-// One 1024-thread workgroup routes all M tokens (a wave per token, 16 at a time) and buckets
-// the (token, slot) pairs by expert. NPL = experts per lane (E <= 64 * NPL).
-// Top-k: k rounds of a wave-wide maximum over the routing keys; slot j holds the j-th largest
-// (ties to the smaller id), the order of the reference's descending sort.
+// One wave routes token t: top-k by k rounds of a wave-wide maximum over the routing keys; slot j
+// holds the j-th largest (ties to the smaller id), the order of the reference's descending sort.
+// NPL = experts per lane (E <= 64 * NPL). pair_e (nullable): the experts in LDS, for the bucketing.
 template <int NPL>
-__global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(const RouteArgs a) {
-  extern __shared__ int lds[];
-  int* pair_e = lds;                                                 // [M*k]
-  int* counts = lds + a.M * a.k;                                     // [kRouteThreads]
-  u32* tmask = reinterpret_cast<u32*>(counts + kRouteThreads);       // [2][kRouteThreads] bits of 64 tokens
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int P = a.M * a.k;
-
-  counts[threadIdx.x] = 0;
-
-  for (int t = wave; t < a.M; t += kRouteThreads / 64) {
-    float xv[NPL];
-    u32 key[NPL];
-    u32 kmax = 0;
-    u16 lg[NPL];  // every lane's logits requested together (clamped index, no branch)
+__device__ __forceinline__ void route_token(const RouteArgs& a, int t, int lane, int* pair_e) {
+  float xv[NPL];
+  u32 key[NPL];
+  u32 kmax = 0;
+  u16 lg[NPL];  // every lane's logits requested together (clamped index, no branch)
 #pragma unroll
-    for (int i = 0; i < NPL; ++i) lg[i] = a.logits[(long)t * a.E + min(lane + 64 * i, a.E - 1)];
+  for (int i = 0; i < NPL; ++i) lg[i] = a.logits[(long)t * a.E + min(lane + 64 * i, a.E - 1)];
 #pragma unroll
-    for (int i = 0; i < NPL; ++i) {
-      const int e = lane + 64 * i;
-      const u32 b = (e < a.E) ? (u32)lg[i] : 0xFF80u;
-      key[i] = (e < a.E) ? route_key(b, e) : 0u;  // every real key is > 0
-      xv[i] = route_key_logit(key[i]);
-      kmax = max(kmax, key[i]);
+  for (int i = 0; i < NPL; ++i) {
+    const int e = lane + 64 * i;
+    const u32 b = (e < a.E) ? (u32)lg[i] : 0xFF80u;
+    key[i] = (e < a.E) ? route_key(b, e) : 0u;  // every real key is > 0
+    xv[i] = route_key_logit(key[i]);
+    kmax = max(kmax, key[i]);
+  }
+  u32 m = wave_max_u32(kmax);
+  const float mx = route_key_logit(m);
+  float sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < NPL; ++i)
+    if (lane + 64 * i < a.E) sum += expf(xv[i] - mx);
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) sum += shfl_xor(sum, o);
+  u32 mine = 0;  // lane j < k keeps the key of slot j
+  for (int j = 0; j < a.k; ++j) {
+    if (j > 0) {
+      kmax = 0;
+#pragma unroll
+      for (int i = 0; i < NPL; ++i) kmax = max(kmax, key[i]);
+      m = wave_max_u32(kmax);
     }
-    u32 m = wave_max_u32(kmax);
-    const float mx = route_key_logit(m);
-    float sum = 0.f;
+    const int e = 0xFFFF - (int)(m & 0xFFFFu);
 #pragma unroll
     for (int i = 0; i < NPL; ++i)
-      if (lane + 64 * i < a.E) sum += expf(xv[i] - mx);
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) sum += shfl_xor(sum, o);
-    u32 mine = 0;  // lane j < k keeps the key of slot j
-    for (int j = 0; j < a.k; ++j) {
-      if (j > 0) {
-        kmax = 0;
-#pragma unroll
-        for (int i = 0; i < NPL; ++i) kmax = max(kmax, key[i]);
-        m = wave_max_u32(kmax);
-      }
-      const int e = 0xFFFF - (int)(m & 0xFFFFu);
-#pragma unroll
-      for (int i = 0; i < NPL; ++i)
-        if (lane + 64 * i == e) key[i] = 0u;
-      if (lane == j) mine = m;
-    }
-    // lanes 0..k-1 finish their slots together: expert, gate value, and the renormalised
-    // score over the slot-order fp32 sum of the k gate values
-    const int e_mine = 0xFFFF - (int)(mine & 0xFFFFu);
-    const float g_mine = bf16r(expf(route_key_logit(mine) - mx) / sum);
-    float gsum = 0.f;
-    for (int j = 0; j < a.k; ++j) gsum += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, g_mine), j));
-    const float denom = bf16r(gsum);
-    if (lane < a.k) {
-      a.inds[t * a.k + lane] = e_mine;
-      pair_e[t * a.k + lane] = e_mine;
-      a.scores[t * a.k + lane] = f2bf(a.renorm ? bf16r(g_mine / denom) : g_mine);
-    }
-    __builtin_amdgcn_wave_barrier();
+      if (lane + 64 * i == e) key[i] = 0u;
+    if (lane == j) mine = m;
   }
-  // the grouped qmm's arrival counters (after the logits loads, which would otherwise wait
-  // behind these stores)
-  for (int i = threadIdx.x; i < a.nctr; i += kRouteThreads) a.ctr[i] = 0;
-  if (!a.offsets) return;
+  // lanes 0..k-1 finish their slots together: expert, gate value, and the renormalised
+  // score over the slot-order fp32 sum of the k gate values
+  const int e_mine = 0xFFFF - (int)(mine & 0xFFFFu);
+  const float g_mine = bf16r(expf(route_key_logit(mine) - mx) / sum);
+  float gsum = 0.f;
+  for (int j = 0; j < a.k; ++j) gsum += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, g_mine), j));
+  const float denom = bf16r(gsum);
+  if (lane < a.k) {
+    a.inds[t * a.k + lane] = e_mine;
+    if (pair_e) pair_e[t * a.k + lane] = e_mine;
+    a.scores[t * a.k + lane] = f2bf(a.renorm ? bf16r(g_mine / denom) : g_mine);
+  }
+}
+
+// Buckets the P = M k (token, slot) pairs of pair_e by expert; one workgroup of kRouteThreads.
+// counts [kRouteThreads] zeroed, pair_e written by any of its threads.
+__device__ __forceinline__ void bucket_pairs(const RouteArgs& a, int* pair_e, int* counts, u32* tmask) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, P = a.M * a.k;
   // ---- bucket the (token, slot) pairs by expert, stable in pair id. A token selects an
   // expert at most once, so a pair's place in its bucket is the number of earlier tokens that
   // selected the same expert. Bucket sizes first (order-free), then an exclusive scan, then
@@ -148,23 +145,33 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(const RouteArg
   // exclusive scan of the bucket sizes by wave 0, 64 experts at a time; counts[e] becomes the
   // bucket start
   if (wave == 0) {
-    int carry = 0;
+    int carry = 0, tcarry = 0;
     for (int c0 = 0; c0 < a.E; c0 += 64) {
       const int e = c0 + lane;
       const int cnt = (e < a.E) ? counts[e] : 0;
-      int incl = cnt;
+      const int nt = a.tiles ? (cnt + a.tile_rows - 1) / a.tile_rows : 0;
+      int incl = cnt, tincl = nt;
 #pragma unroll
       for (int d = 1; d < 64; d <<= 1) {
-        const int o = __shfl_up(incl, d);
-        if (lane >= d) incl += o;
+        const int o = __shfl_up(incl, d), to = __shfl_up(tincl, d);
+        if (lane >= d) {
+          incl += o;
+          tincl += to;
+        }
       }
       if (e < a.E) {
         a.offsets[e] = carry + incl - cnt;
         counts[e] = carry + incl - cnt;
       }
+      for (int i = 0; i < nt; ++i)
+        a.tiles[tcarry + tincl - nt + i] = wide::MoeTile{e, carry + incl - cnt + i * a.tile_rows,
+                                                         min(a.tile_rows, cnt - i * a.tile_rows), 0};
       carry += __shfl(incl, 63);
+      tcarry += __shfl(tincl, 63);
     }
     if (lane == 0) a.offsets[a.E] = carry;
+    if (a.tiles)
+      for (int i = tcarry + lane; i < a.max_tiles; i += 64) a.tiles[i] = wide::MoeTile{0, 0, 0, 0};
   }
   for (int t0 = 0; t0 < a.M; t0 += 64) {
     tmask[threadIdx.x] = 0;
@@ -188,6 +195,41 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(const RouteArg
     __syncthreads();
     counts[threadIdx.x] += __builtin_popcount(tmask[threadIdx.x]) + __builtin_popcount(tmask[kRouteThreads + threadIdx.x]);
   }
+}
+
+// LDS: pair_e [M k], counts [kRouteThreads], tmask [2][kRouteThreads] (bits of 64 tokens)
+constexpr size_t route_lds(size_t pairs) { return sizeof(int) * (pairs + 3 * kRouteThreads); }
+
+// One workgroup routes all M tokens (a wave per token, 16 at a time) and buckets the pairs.
+template <int NPL>
+__global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(const RouteArgs a) {
+  extern __shared__ int lds[];
+  int* counts = lds + a.M * a.k;
+  counts[threadIdx.x] = 0;
+  for (int t = threadIdx.x >> 6; t < a.M; t += kRouteThreads / 64) {
+    route_token<NPL>(a, t, threadIdx.x & 63, lds);
+    __builtin_amdgcn_wave_barrier();
+  }
+  // the grouped qmm's arrival counters (after the logits loads, which would otherwise wait
+  // behind these stores)
+  for (int i = threadIdx.x; i < a.nctr; i += kRouteThreads) a.ctr[i] = 0;
+  if (a.offsets) bucket_pairs(a, lds, counts, reinterpret_cast<u32*>(counts + kRouteThreads));
+}
+
+// Many tokens: a wave per token over the whole chip, then one workgroup for the buckets.
+template <int NPL>
+__global__ __launch_bounds__(256) void moe_topk_kernel(const RouteArgs a) {
+  const int t = blockIdx.x * 4 + uniform(threadIdx.x >> 6);
+  if (t < a.M) route_token<NPL>(a, t, threadIdx.x & 63, nullptr);
+}
+
+__global__ __launch_bounds__(kRouteThreads) void moe_bucket_kernel(const RouteArgs a) {
+  extern __shared__ int lds[];
+  int* counts = lds + a.M * a.k;
+  counts[threadIdx.x] = 0;
+  for (int p = threadIdx.x; p < a.M * a.k; p += kRouteThreads) lds[p] = a.inds[p];
+  for (int i = threadIdx.x; i < a.nctr; i += kRouteThreads) a.ctr[i] = 0;
+  bucket_pairs(a, lds, counts, reinterpret_cast<u32*>(counts + kRouteThreads));
 }
 
 // ---------------------------------------------------------------- grouped expert qmm
@@ -359,14 +401,23 @@ int check_route(long M, long E, long k) {
   return DSPARK_OK;
 }
 
+template <int NPL>
+void launch_route_n(const RouteArgs& a, hipStream_t s) {
+  const size_t lds = route_lds((size_t)a.M * a.k);
+  if (a.M <= kRouteOneGroup) {
+    hipLaunchKernelGGL(moe_route_kernel<NPL>, dim3(1), dim3(kRouteThreads), lds, s, a);
+    return;
+  }
+  hipLaunchKernelGGL(moe_topk_kernel<NPL>, dim3((unsigned)((a.M + 3) / 4)), dim3(256), 0, s, a);
+  if (a.offsets) hipLaunchKernelGGL(moe_bucket_kernel, dim3(1), dim3(kRouteThreads), lds, s, a);
+}
+
 int launch_route(const RouteArgs& a, hipStream_t s) {
-  const size_t lds = sizeof(int) * ((size_t)a.M * a.k + 3 * kRouteThreads);
-  const dim3 g(1), b(kRouteThreads);
-  if (a.E <= 64) hipLaunchKernelGGL(moe_route_kernel<1>, g, b, lds, s, a);
-  else if (a.E <= 128) hipLaunchKernelGGL(moe_route_kernel<2>, g, b, lds, s, a);
-  else if (a.E <= 256) hipLaunchKernelGGL(moe_route_kernel<4>, g, b, lds, s, a);
-  else if (a.E <= 512) hipLaunchKernelGGL(moe_route_kernel<8>, g, b, lds, s, a);
-  else hipLaunchKernelGGL(moe_route_kernel<16>, g, b, lds, s, a);
+  if (a.E <= 64) launch_route_n<1>(a, s);
+  else if (a.E <= 128) launch_route_n<2>(a, s);
+  else if (a.E <= 256) launch_route_n<4>(a, s);
+  else if (a.E <= 512) launch_route_n<8>(a, s);
+  else launch_route_n<16>(a, s);
   return check_launch("moe_route_topk");
 }
 
@@ -424,11 +475,24 @@ MoePlan moe_plan(long K, long N, long E, long M, bool swiglu, int bits) {
 }
 
 struct MoeWorkspace {
-  size_t offsets, sorted, pos, inds, scores, h, y, ctr, part, total;
+  size_t offsets, sorted, pos, inds, scores, h, y, ctr, part, tiles, xsums, hsums, total;
   MoePlan gu, dn;
+  int wide_mt, max_tiles;  // large buckets: 16-row tiles of a workgroup, 0 for the small-bucket kernels
+  int gp_x, gp_h;
 };
 
-// (bits only picks the kernel instantiation; the sizes do not depend on it)
+// Whether the buckets are large enough for the grouped prefill product (dspark_moe_wide.h), which
+// reads an expert's weights once for 32 or 64 rows, where the small-bucket kernels take 4 rows a pass
+// and 16 a workgroup. Its longer beginning and end cost small experts more. Measured, small-bucket /
+// grouped: 128 experts top 8, 2048 x 768, 4 bits: 3 rows a bucket 106 / 132 us, 4 rows 140 / 132, 32
+// rows 566 / 196; 8 bits: 3 rows 139 / 164, 4 rows 174 / 166; 32 experts top 4, 1024 x 384: 6 rows
+// 31.5 / 42.5, 8 rows 44.2 / 43.8, 16 rows 63 / 45.
+bool moe_wide(long M, long H, long I, long E, long k) {
+  const long rows = E * H * I >= 1L << 26 ? 4 : 8;
+  return M > 16 && M * k >= rows * E;
+}
+
+// (of both widths 4 bits need no less: their row tiles are no taller, so no fewer)
 MoeWorkspace moe_layout(long M, long H, long I, long E, long k, int bits) {
   MoeWorkspace w{};
   w.gu = moe_plan(H, I, E, M, true, bits);
@@ -444,6 +508,16 @@ MoeWorkspace moe_layout(long M, long H, long I, long E, long k, int bits) {
   w.y = o;       o += align256(sizeof(u16) * P * H);
   w.ctr = o;     o += align256(sizeof(int) * (w.gu.ctrs > w.dn.ctrs ? w.gu.ctrs : w.dn.ctrs));
   w.part = o;    o += align256(sizeof(float) * (w.gu.part_floats > w.dn.part_floats ? w.gu.part_floats : w.dn.part_floats));
+  w.gp_x = (int)((H / 64 + 31) / 32 * 32);
+  w.gp_h = (int)((I / 64 + 31) / 32 * 32);
+  if (moe_wide(M, H, I, E, k)) {
+    w.wide_mt = moe_wide_mt((long)P, E, bits);
+    // sum over experts of ceil(rows / tile) <= P / tile + the experts that have rows
+    w.max_tiles = (int)(P / (16 * w.wide_mt) + std::min((size_t)E, P));
+    w.tiles = o;   o += align256(sizeof(wide::MoeTile) * w.max_tiles);
+    w.xsums = o;   o += align256(sizeof(u16) * wide::kPieces * M * w.gp_x);
+    w.hsums = o;   o += align256(sizeof(u16) * wide::kPieces * P * w.gp_h);
+  }
   w.total = o;
   return w;
 }
@@ -657,6 +731,13 @@ int switch_glu_impl(const void* x, const void* logits, int64_t M, int64_t H, int
   u16* ypair = reinterpret_cast<u16*>(ws + L.y);
   hipStream_t s = static_cast<hipStream_t>(stream);
 
+  const RcPlan rgu = rc_plan(H, I, true, s_gate, b_gate), rgu2 = rc_plan(H, I, true, s_up, b_up);
+  const RcPlan rdn = rc_plan(I, H, false, s_down, b_down);
+  if (packed && (!rgu.kw || !rgu2.kw || !rdn.kw))
+    return fail(DSPARK_ERR_UNSUPPORTED,
+                "moe_switch_glu_packed: H=%lld I=%lld need K %% 128 == 0 and 16-byte aligned scales and biases",
+                (long long)H, (long long)I);
+
   RouteArgs r{};
   r.logits = static_cast<const u16*>(logits);
   r.inds = inds_ws;
@@ -671,9 +752,52 @@ int switch_glu_impl(const void* x, const void* logits, int64_t M, int64_t H, int
   int* ctr = reinterpret_cast<int*>(ws + L.ctr);
   r.ctr = ctr;  // the grouped qmm's arrival counters start every block at zero
   r.nctr = (int)(L.gu.ctrs > L.dn.ctrs ? L.gu.ctrs : L.dn.ctrs);
+  if (L.wide_mt) {
+    r.tiles = reinterpret_cast<wide::MoeTile*>(ws + L.tiles);
+    r.tile_rows = 16 * L.wide_mt;
+    r.max_tiles = L.max_tiles;
+    r.nctr = 0;
+  }
   if ((st = launch_route(r, s))) return st;
 
   const int P = (int)(M * k);
+  auto combine = [&] {
+    hipLaunchKernelGGL(moe_combine_kernel, dim3((unsigned)M, (unsigned)((H + 255) / 256)), dim3(256), 0, s, ypair, pos,
+                       scores_ws, static_cast<u16*>(out), (int)H, (int)k);
+    return check_launch("moe combine");
+  };
+  if (L.wide_mt) {
+    wide::MoeWideArgs g{};
+    g.x = static_cast<const u16*>(x);
+    g.xs = reinterpret_cast<u16*>(ws + L.xsums);
+    g.row_index = sorted;
+    g.tiles = r.tiles;
+    g.w[0] = reinterpret_cast<const char*>(w_gate), g.w[1] = reinterpret_cast<const char*>(w_up);
+    g.s[0] = static_cast<const u16*>(s_gate), g.s[1] = static_cast<const u16*>(s_up);
+    g.b[0] = static_cast<const u16*>(b_gate), g.b[1] = static_cast<const u16*>(b_up);
+    g.y = h;
+    g.ldx = H, g.ldy = I, g.nrows = M;
+    g.K = (int)H, g.N = (int)I, g.G = (int)(H / 64), g.GP = L.gp_x;
+    g.row_div = (int)k;
+    g.max_tiles = L.max_tiles;
+    g.vec = wide::chunk_rows(g.G, s_gate, b_gate) && wide::chunk_rows(g.G, s_up, b_up);
+    if ((st = wide::launch_group_sums(g.x, H, M, g.G, g.GP, const_cast<u16*>(g.xs), s))) return st;
+    if ((st = launch_moe_wide(g, true, packed, L.wide_mt, bits, s))) return st;
+    wide::MoeWideArgs d = g;
+    d.x = h;
+    d.xs = reinterpret_cast<u16*>(ws + L.hsums);
+    d.row_index = nullptr;
+    d.w[0] = d.w[1] = reinterpret_cast<const char*>(w_down);
+    d.s[0] = d.s[1] = static_cast<const u16*>(s_down);
+    d.b[0] = d.b[1] = static_cast<const u16*>(b_down);
+    d.y = ypair;
+    d.ldx = I, d.ldy = H, d.nrows = P;
+    d.K = (int)I, d.N = (int)H, d.G = (int)(I / 64), d.GP = L.gp_h;
+    d.vec = wide::chunk_rows(d.G, s_down, b_down);
+    if ((st = wide::launch_group_sums(h, I, P, d.G, d.GP, const_cast<u16*>(d.xs), s))) return st;
+    if ((st = launch_moe_wide(d, false, packed, L.wide_mt, bits, s))) return st;
+    return combine();
+  }
   float* part = reinterpret_cast<float*>(ws + L.part);
   MoeSkArgs g{};
   g.x = static_cast<const u16*>(x);
@@ -697,12 +821,6 @@ int switch_glu_impl(const void* x, const void* logits, int64_t M, int64_t H, int
   g.strips = L.gu.strips;
   g.mtiles = L.gu.mtiles;
   g.S = L.gu.S;
-  const RcPlan rgu = rc_plan(H, I, true, s_gate, b_gate), rgu2 = rc_plan(H, I, true, s_up, b_up);
-  const RcPlan rdn = rc_plan(I, H, false, s_down, b_down);
-  if (packed && (!rgu.kw || !rgu2.kw || !rdn.kw))
-    return fail(DSPARK_ERR_UNSUPPORTED,
-                "moe_switch_glu_packed: H=%lld I=%lld need K %% 128 == 0 and 16-byte aligned scales and biases",
-                (long long)H, (long long)I);
   if (packed && moe_cu_gate_up(M, H, I, E, k, bits)) {
     if ((st = launch_moe_cu(cu_args(g, sorted, M, E, k, bits), H, bits, s))) return st;
   } else if (packed) {
@@ -740,9 +858,7 @@ int switch_glu_impl(const void* x, const void* logits, int64_t M, int64_t H, int
     return st;
   }
 
-  hipLaunchKernelGGL(moe_combine_kernel, dim3((unsigned)M, (unsigned)((H + 255) / 256)), dim3(256), 0, s, ypair, pos,
-                     scores_ws, static_cast<u16*>(out), (int)H, (int)k);
-  return check_launch("moe combine");
+  return combine();
 }
 }  // namespace
 }  // namespace dspark

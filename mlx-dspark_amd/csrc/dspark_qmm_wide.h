@@ -65,11 +65,15 @@ struct Raw<4> {
   u32x2_t v;
 };
 
+// x copies of a wave per group: 8 rows each, 32 of the workgroup's
+template <int MT>
+constexpr int kCopies = (MT + 1) / 2;
+
 // Everything of a tile that does not depend on the group.
 template <int MT, int NT>
 struct Tile {
   const char* xb;        // x, the base of the row offsets
-  u32 xoff[MT / 2];      // byte offset of this lane's 16-byte chunk of each x copy it issues
+  u32 xoff[kCopies<MT>];      // byte offset of this lane's 16-byte chunk of each x copy it issues
   const u16* xs;         // group-sum pieces
   u32 xsoff[MT];         // element offset of this lane's row of every row tile
   long xs_piece;         // elements between pieces
@@ -79,8 +83,11 @@ struct Tile {
   const u16* brow[NT];   // this lane's bias rows
   const u16* sown[NT];   // this lane's scale rows (the 4-bit offset term)
   int G, gs, ge;
-  bool vec;              // scale / bias rows are whole aligned 16-byte chunks (G % 8 == 0)
+  bool vec;              // scale / bias rows are whole aligned 16-byte chunks (chunk_rows)
 };
+
+// Whether rows of G scales and biases are whole aligned 16-byte chunks
+inline bool chunk_rows(int G, const void* s, const void* b) { return G % 8 == 0 && aligned(s, 16) && aligned(b, 16); }
 
 template <int BITS, bool PW>
 __device__ __forceinline__ u32 w_step(int g) {  // byte offset of group g along a row / packed tile
@@ -88,15 +95,27 @@ __device__ __forceinline__ u32 w_step(int g) {  // byte offset of group g along 
   else return (u32)g * (BITS == 8 ? 64u : 32u);
 }
 
-// 8 consecutive bf16 of a row of G starting at g0, zeros past its end
+// Rows that are not whole 16-byte chunks are read as the aligned words that hold them: word i of a
+// row holds its elements 2 i - odd_start and the next
+__device__ __forceinline__ int odd_start(const u16* row) { return (int)(reinterpret_cast<uintptr_t>(row) >> 1) & 1; }
+__device__ __forceinline__ const u32* row_words(const u16* row) {
+  return reinterpret_cast<const u32*>(reinterpret_cast<uintptr_t>(row) & ~(uintptr_t)3);
+}
+
+// 8 consecutive bf16 of a row of G starting at g0 (a multiple of 8), zeros past its end
 __device__ __forceinline__ u32x4_t row8(const u16* row, int g0, int G, bool vec) {
   if (vec) return g0 < G ? ldg128(row + g0) : u32x4_t{0u, 0u, 0u, 0u};
+  const int odd = odd_start(row), last = (odd + G - 1) >> 1;
+  const u32* p = row_words(row);
+  u32 w[5];
+#pragma unroll
+  for (int i = 0; i < 5; ++i) w[i] = p[min((g0 >> 1) + i, last)];
   u32x4_t o;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int a = g0 + 2 * i;
-    const u32 lo = row[min(a, G - 1)], hi = row[min(a + 1, G - 1)];
-    o[i] = (a < G ? lo : 0u) | ((a + 1 < G ? hi : 0u) << 16);
+    const u32 v = __builtin_amdgcn_alignbit(w[i + 1], w[i], 16 * odd);
+    o[i] = a + 1 < G ? v : a < G ? v & 0xFFFFu : 0u;
   }
   return o;
 }
@@ -117,7 +136,7 @@ constexpr int kAhead = MT * NT >= 24 ? 1 : 3;
 
 template <int MT, int NT>
 struct __attribute__((aligned(16))) Smem {
-  u16 xa[kAhead<MT, NT> + 1][16 * MT * 64];
+  u16 xa[kAhead<MT, NT> + 1][32 * kCopies<MT> * 64];
   u16 sc[2][kThreads * 8];
 };
 
@@ -137,9 +156,9 @@ __device__ __forceinline__ void tile_loop(const Tile<MT, NT>& t, Smem<MT, NT>& s
 
   auto copy_x = [&](int g, int buf) {
 #pragma unroll
-    for (int j = 0; j < MT / 2; ++j)
+    for (int j = 0; j < kCopies<MT>; ++j)
       __builtin_amdgcn_global_load_lds((glb_u16*)(t.xb + (size_t)g * 128 + t.xoff[j]),
-                                       (lds_u16*)&sm.xa[buf][(wave * (MT / 2) + j) * 512], 16, 0, 0);
+                                       (lds_u16*)&sm.xa[buf][(wave * kCopies<MT> + j) * 512], 16, 0, 0);
   };
   auto load_w = [&](int g, Raw<BITS> (&raw)[NT]) {
 #pragma unroll
@@ -186,14 +205,14 @@ __device__ __forceinline__ void tile_loop(const Tile<MT, NT>& t, Smem<MT, NT>& s
   }
 
   if (tid < 64 * NT) *reinterpret_cast<u32x4_t*>(&sm.sc[(t.gs >> 3) & 1][tid * 8]) = scn;
-  const int abase = c16 * 64 + ((k_chunk<BITS>(q) ^ (c16 & 7)) << 3);  // the second chunk: ^ 8
+  const int abase = c16 * 64 + ((k_chunk<BITS>(q) ^ ((c16 >> 1) & 7)) << 3);  // the second chunk: ^ 8
   const int sbase = (wave * 16 * NT + c16) * 8;
   int buf = 0;
   auto step = [&](int g, Raw<BITS> (&rw)[NT]) {
     // x tile g and the staged scales are in LDS once every wave's copies have landed; the loads
     // of the PD - 1 groups after g stay in flight over the barrier (a __syncthreads would wait
     // for them). Every LDS read of the step before has been used by then.
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((PD - 1) * (NT + MT / 2)) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((PD - 1) * (NT + kCopies<MT>)) : "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     u32x4_t b[NT][2];
@@ -267,12 +286,13 @@ __device__ __forceinline__ void tile_loop(const Tile<MT, NT>& t, Smem<MT, NT>& s
 }
 
 // This thread's chunk of the x copies: LDS chunk l of copy j lies in tile row 8 (..) + (l >> 3);
-// row r holds its eight 16-byte chunks in the order chunk ^ (r & 7).
+// row r holds its eight 16-byte chunks in the order chunk ^ ((r >> 1) & 7), which with the row's
+// parity spreads 16 rows read at one chunk over the banks.
 template <int MT>
 __device__ __forceinline__ int copy_row(int j) {
-  return 8 * ((int)(threadIdx.x >> 6) * (MT / 2) + j) + ((threadIdx.x & 63) >> 3);
+  return 8 * ((int)(threadIdx.x >> 6) * kCopies<MT> + j) + ((threadIdx.x & 63) >> 3);
 }
-__device__ __forceinline__ int copy_chunk(int row) { return (threadIdx.x & 7) ^ (row & 7); }
+__device__ __forceinline__ int copy_chunk(int row) { return (threadIdx.x & 7) ^ ((row >> 1) & 7); }
 
 // ---------------------------------------------------------------- the dense matrix
 
@@ -340,7 +360,7 @@ __global__ __launch_bounds__(kThreads, 2) void wide_kernel(const Args a) {
   t.xb = reinterpret_cast<const char*>(a.x + (long)m0 * a.ldx);
   const int mlast = a.M - 1 - m0;  // rows past M repeat the last one; their outputs are dropped
 #pragma unroll
-  for (int j = 0; j < MT / 2; ++j) {
+  for (int j = 0; j < kCopies<MT>; ++j) {
     const int r = copy_row<MT>(j);
     t.xoff[j] = (u32)(min(r, mlast) * (int)a.ldx * 2 + copy_chunk(r) * 16);
   }
@@ -426,32 +446,8 @@ __global__ __launch_bounds__(256) void wide_reduce_kernel(const Args a) {
   }
 }
 
-// Group sums of x as bf16 pieces: xs[p][m][g], sum = piece 0 + piece 1 + piece 2 to 24 bits (the
-// fp32 sum); zeros for g in [G, GP). 8 lanes a (row, group).
-__global__ __launch_bounds__(256) void wide_xsum_kernel(const u16* __restrict__ x, long ldx, int M, int G, int GP,
-                                                        u16* __restrict__ xs) {
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  const long rg = i >> 3;
-  if (rg >= (long)M * GP) return;  // whole 8-lane groups leave together
-  const int m = (int)(rg / GP), g = (int)(rg - (long)m * GP);
-  float s = 0.f;
-  if (g < G) {
-    const u32x4_t v = ldg128(x + (long)m * ldx + 64 * g + 8 * (i & 7));
-#pragma unroll
-    for (int j = 0; j < 4; ++j) s += bf2f(v[j] & 0xFFFFu) + bf2f(v[j] >> 16);
-  }
-  s = sum8_lanes(s);
-  if ((i & 7) == 0) {
-    const u16 h = f2bf(s);
-    const float r1 = s - bf2f(h);
-    const u16 mid = f2bf(r1);
-    const u16 lo = f2bf(r1 - bf2f(mid));
-    const long piece = (long)M * GP, o = (long)m * GP + g;
-    xs[o] = h;
-    xs[o + piece] = mid;
-    xs[o + 2 * piece] = lo;
-  }
-}
+// Group sums of x [M, K = 64 G] as bf16 pieces xs[p][m][g], rows of GP entries (g >= G zero)
+int launch_group_sums(const u16* x, long ldx, long M, int G, int GP, u16* xs, hipStream_t s);
 
 }  // namespace wide
 }  // namespace dspark

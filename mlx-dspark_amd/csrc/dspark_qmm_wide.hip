@@ -7,6 +7,33 @@ namespace dspark {
 namespace wide {
 namespace {
 
+// Group sums of x as bf16 pieces: xs[p][m][g], sum = piece 0 + piece 1 + piece 2 to 24 bits (the
+// fp32 sum); zeros for g in [G, GP). 8 lanes a (row, group).
+__global__ __launch_bounds__(256) void wide_xsum_kernel(const u16* __restrict__ x, long ldx, int M, int G, int GP,
+                                                        u16* __restrict__ xs) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  const long rg = i >> 3;
+  if (rg >= (long)M * GP) return;  // whole 8-lane groups leave together
+  const int m = (int)(rg / GP), g = (int)(rg - (long)m * GP);
+  float s = 0.f;
+  if (g < G) {
+    const u32x4_t v = ldg128(x + (long)m * ldx + 64 * g + 8 * (i & 7));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s += bf2f(v[j] & 0xFFFFu) + bf2f(v[j] >> 16);
+  }
+  s = sum8_lanes(s);
+  if ((i & 7) == 0) {
+    const u16 h = f2bf(s);
+    const float r1 = s - bf2f(h);
+    const u16 mid = f2bf(r1);
+    const u16 lo = f2bf(r1 - bf2f(mid));
+    const long piece = (long)M * GP, o = (long)m * GP + g;
+    xs[o] = h;
+    xs[o + piece] = mid;
+    xs[o + 2 * piece] = lo;
+  }
+}
+
 struct Plan {
   int mt, nt, S;            // 16-row tiles and 16-column tiles per wave, K slices
   int mtiles, ntiles;
@@ -74,6 +101,14 @@ void launch(const Args& a, int mt, unsigned blocks, hipStream_t s) {
 }
 
 }  // namespace
+
+int launch_group_sums(const u16* x, long ldx, long M, int G, int GP, u16* xs, hipStream_t s) {
+  const long threads = M * GP * 8;
+  hipLaunchKernelGGL(wide_xsum_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, x, ldx, (int)M, G, GP,
+                     xs);
+  return check_launch("qmm_wide group sums");
+}
+
 }  // namespace wide
 }  // namespace dspark
 
@@ -119,15 +154,12 @@ extern "C" int dspark_qmm_wide(const void* x, int64_t ldx, int64_t M, int64_t K,
   a.S = p.S;
   a.mtiles = p.mtiles;
   a.ntiles = p.ntiles;
-  a.vec = a.G % 8 == 0 && aligned(scales, 16) && aligned(biases, 16);
+  a.vec = wide::chunk_rows(a.G, scales, biases);
   const long tiles = (long)p.mtiles * p.ntiles * p.S;
   if (tiles > (1L << 30)) return fail(DSPARK_ERR_SHAPE, "qmm_wide: too many tiles");
   a.per_xcd = (int)((tiles + 7) / 8);
 
-  const long sums = (long)M * p.GP * 8;
-  hipLaunchKernelGGL(wide::wide_xsum_kernel, dim3((unsigned)((sums + 255) / 256)), dim3(256), 0, s, a.x, (long)ldx,
-                     a.M, a.G, p.GP, xs);
-  if ((st = check_launch("qmm_wide group sums"))) return st;
+  if ((st = wide::launch_group_sums(a.x, ldx, M, a.G, p.GP, xs, s))) return st;
   const unsigned blocks = (unsigned)a.per_xcd * 8;
   if (bits == 8) {
     if (p.nt == 4) wide::launch<8, 4>(a, p.mt, blocks, s);
