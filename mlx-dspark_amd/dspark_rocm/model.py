@@ -73,6 +73,34 @@ def rope(x: torch.Tensor, pos0: int, base: float) -> torch.Tensor:
     return torch.cat([(x1 * c - x2 * s).to(torch.bfloat16), (x1 * s + x2 * c).to(torch.bfloat16)], dim=-1)
 
 
+FUSED_MIN_ROWS = 17     # rows from which the module path takes the fused row kernels (prefill widths)
+
+
+def _fused(rows: int, *ts: torch.Tensor) -> bool:
+    """Whether the fused row kernels (``ops.rmsnorm``, ``qk_norm_rope_kv``, ``swiglu``: the torch ops'
+    rounding points in one pass each) may take a call of ``rows`` rows on these tensors: prefill
+    widths of plain contiguous bf16 tensors on the GPU, nothing recording gradients. A verify block's
+    module path keeps the torch ops the engine is checked against."""
+    return (FUSED_MIN_ROWS <= rows <= 65535 and ops.eager_inference(*ts)
+            and ts[0].device.index == torch.cuda.current_device()
+            and all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.shape[-1] % 8 == 0
+                    and t.data_ptr() % 16 == 0 for t in ts))
+
+
+def add_rms_norm(x: torch.Tensor, r: torch.Tensor | None, w: torch.Tensor, eps: float):
+    """(h, rms_norm(h, w)) of h = x + r (x alone without r)."""
+    rows = x.numel() // max(x.shape[-1], 1)
+    if w.shape == x.shape[-1:] and (r is None or r.shape == x.shape) \
+            and _fused(rows, *((x, w) if r is None else (x, r, w))):
+        x2 = x.view(rows, -1)
+        h = x if r is None else torch.empty_like(x)
+        y = ops.rmsnorm(x2, w, eps, residual=None if r is None else r.view(rows, -1),
+                        h_out=None if r is None else h.view(rows, -1))
+        return h, y.view(x.shape)
+    h = x if r is None else x + r
+    return h, rms_norm(h, w, eps)
+
+
 class Attention(nn.Module):
     def __init__(self, args: ModelArgs, q, k, v, o, q_norm, k_norm):
         super().__init__()
@@ -85,12 +113,22 @@ class Attention(nn.Module):
         a = self.args
         B, L, _ = x.shape
         hq, hk, d = a.num_attention_heads, a.num_key_value_heads, a.head_dim
-        q = rms_norm(self.q_proj(x).reshape(B, L, hq, d), self.q_norm, a.rms_norm_eps).transpose(1, 2)
-        k = rms_norm(self.k_proj(x).reshape(B, L, hk, d), self.k_norm, a.rms_norm_eps).transpose(1, 2)
-        v = self.v_proj(x).reshape(B, L, hk, d).transpose(1, 2)
-        q = rope(q, cache.offset, a.rope_theta)
-        k = rope(k, cache.offset, a.rope_theta)
-        keys, values = cache.update_and_fetch(k, v)
+        q, k, v = self.q_proj(x), self.k_proj(x), self.v_proj(x)
+        if self._fused_kv(q, k, v, cache):
+            cache.reserve(L)
+            q = ops.qk_norm_rope_kv(q[0], k[0], v[0], self.q_norm, self.k_norm, heads=hq, kv_heads=hk, head_dim=d,
+                                    eps=a.rms_norm_eps, rope_base=a.rope_theta, pos0=cache.offset,
+                                    q_out=q.new_empty((hq, L, d)), k_cache=cache.keys[0],
+                                    v_cache=cache.values[0]).unsqueeze(0)
+            cache.advance(L)
+            keys, values = cache.fetch()
+        else:
+            q = rms_norm(q.reshape(B, L, hq, d), self.q_norm, a.rms_norm_eps).transpose(1, 2)
+            k = rms_norm(k.reshape(B, L, hk, d), self.k_norm, a.rms_norm_eps).transpose(1, 2)
+            v = v.reshape(B, L, hk, d).transpose(1, 2)
+            q = rope(q, cache.offset, a.rope_theta)
+            k = rope(k, cache.offset, a.rope_theta)
+            keys, values = cache.update_and_fetch(k, v)
         mask = "causal" if L > 1 else None
         if hasattr(cache, "bits"):
             # mlx-lm's attention helper dispatches per cache: a quantized cache takes
@@ -103,14 +141,32 @@ class Attention(nn.Module):
         return self.o_proj(out.transpose(1, 2).reshape(B, L, hq * d))
 
 
+    def _fused_kv(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cache) -> bool:
+        """Whether one launch norms and rotates q and k and writes k and v into a plain bf16 cache."""
+        a = self.args
+        hq, hk, d = a.num_attention_heads, a.num_key_value_heads, a.head_dim
+        if type(cache) is not KVCache or q.dim() != 3 or q.shape[0] != 1 or d % 8 or not 8 <= d <= 256:
+            return False
+        L = q.shape[1]
+        return (tuple(q.shape) == (1, L, hq * d) and tuple(k.shape) == tuple(v.shape) == (1, L, hk * d)
+                and cache.keys.shape[:2] == (1, hk) and cache.keys.shape[3] == d
+                and self.q_norm.shape == self.k_norm.shape == (d,)
+                and _fused(L, q, k, v, self.q_norm, self.k_norm, cache.keys, cache.values))
+
+
 class MLP(nn.Module):
     def __init__(self, gate, up, down):
         super().__init__()
         self.gate_proj, self.up_proj, self.down_proj = gate, up, down
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        g = self.gate_proj(x)
-        return self.down_proj((g * torch.sigmoid(g)) * self.up_proj(x))
+        g, u = self.gate_proj(x), self.up_proj(x)
+        rows = g.numel() // max(g.shape[-1], 1)
+        if g.shape == u.shape and _fused(rows, g, u):
+            h = ops.swiglu(g.view(rows, -1), u.view(rows, -1)).view(g.shape)
+        else:
+            h = (g * torch.sigmoid(g)) * u
+        return self.down_proj(h)
 
 
 class DecoderLayer(nn.Module):
@@ -123,8 +179,9 @@ class DecoderLayer(nn.Module):
 
     def forward(self, x: torch.Tensor, cache: KVCache) -> torch.Tensor:
         eps = self.args.rms_norm_eps
-        h = x + self.self_attn(rms_norm(x, self.input_layernorm, eps), cache)
-        return h + self.mlp(rms_norm(h, self.post_attention_layernorm, eps))
+        x, y = add_rms_norm(x, None, self.input_layernorm, eps)
+        h, y = add_rms_norm(x, self.self_attn(y, cache), self.post_attention_layernorm, eps)
+        return h + self.mlp(y)
 
 
 class DenseModel(nn.Module):
@@ -186,7 +243,7 @@ class DenseModel(nn.Module):
         fused = None
         if tap is not None:
             fused = torch.cat(captured, dim=-1) if captured else h.new_empty((*h.shape[:-1], 0))
-        return rms_norm(h, self.norm, self.args.rms_norm_eps), fused
+        return add_rms_norm(h, None, self.norm, self.args.rms_norm_eps)[1], fused
 
     def forward(self, ids: torch.Tensor, cache: list[KVCache]) -> torch.Tensor:
         """ids [1, L] -> logits [1, L, V] (the module path)."""

@@ -132,10 +132,12 @@ def _bars(bits: int) -> list[gate.Bar]:
 
 
 def _race(mods: list, rows: int, gen: torch.Generator) -> float:
-    """Stock / kernel time at ``rows`` rows over chains rotating through ``mods``."""
+    """Dequantized product / kernel time at ``rows`` rows over chains rotating through ``mods``: the
+    bars were set for it (the stock path's own matrix-core product is built for prefill widths and
+    behind these kernels in all of their window)."""
     x = _probe_x(_in_features(mods[0]), rows, gen, mods[0].weight.device)
     seq = [mods[t % len(mods)] for t in range(_CHAIN)]
-    return gate.speedup([lambda m=m: _orig_call(m, x) for m in seq],
+    return gate.speedup([lambda m=m: m.torch_product(x) for m in seq],
                         [lambda m=m: _kernel_rows(m, x) for m in seq], repeat=_EVALS - 1)
 
 

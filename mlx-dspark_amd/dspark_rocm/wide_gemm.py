@@ -6,7 +6,7 @@ the product of the leading dims, so a ``[1, L, K]`` prefill counts L) whose shap
 verified allowlist takes the wide path, and the result is **bit-identical** to the stock path
 for that shape; everything else runs the forward installed on entry, unchanged.
 
-What the wide path replaces here. bf16 calls of more than 16 rows never see it: there the stock
+What the wide path replaces here. bf16 calls never see it: there the stock
 path is already the matrix-core product over the packed weight (:meth:`QuantizedLinear.wide_kernel`),
 and :func:`wide_rows` makes the same call, so the bits agree. For the other activation and scale
 dtypes the stock path dequantizes with torch elementwise ops -- unpack through int64, convert,
