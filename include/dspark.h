@@ -523,6 +523,43 @@ int dspark_qk_norm_rope_kv_quantized(const void* q, int64_t ldq, const void* k, 
 int dspark_swiglu(const void* g, int64_t ldg, const void* u, int64_t ldu, int64_t M, int64_t N, void* h,
                   int64_t ldh, dspark_stream stream);
 
+/*
+ * The launches of one verify step of a dense target (target.py:642-677 -> :187-221, :347-354) over
+ * packed weights, in one call: per layer residual add + RMSNorm, q/k/v, q/k norm + RoPE + cache
+ * write, attention, o, residual add + RMSNorm, gate / up / SwiGLU, down; then the final norm and the
+ * head. Exactly the entry points above in that order, with their checks; the first failing one's
+ * status is returned. h [M, H] holds the embedded rows on entry. Every field of both structs is 8
+ * bytes wide. Row-major buffers of M rows: h, y, r [H], q and att [Hq*D], k and v [Hk*D], hm [I],
+ * logits [vocab]; qatt [Hq, M, D].
+ */
+typedef struct dspark_verify_args {
+  int64_t M, H, I, Hq, Hk, D, pos0, kv_bits; /* kv_bits 0: bf16 caches */
+  double eps, rope_base, scale;
+  void *h, *y, *r, *q, *k, *v, *qatt, *att, *hm;
+  void* qmm_ws;
+  int64_t qmm_ws_bytes;
+  void* attn_ws;
+  int64_t attn_ws_bytes;
+  const void *final_norm, *head;
+  int64_t head_bits, vocab;
+  void* logits;
+} dspark_verify_args;
+
+typedef struct dspark_verify_layer {
+  const void *input_norm, *q_norm, *k_norm, *post_norm;
+  const void *q, *k, *v, *o, *gate_up, *down; /* dspark_qmm_pack / dspark_qmm_pack_swiglu forms */
+  int64_t qkv_bits, o_bits, mlp_bits, down_bits;
+  void *k_cache, *v_cache; /* rows, or words when kv_bits */
+  int64_t k_head, k_pos, v_head, v_pos; /* their strides, in elements (words) */
+  void *k_scales, *k_biases, *v_scales, *v_biases;
+  int64_t ks_head, ks_pos, vs_head, vs_pos;
+  void* stream; /* where the residual stream after the layer goes, rows ld_stream elements apart */
+  int64_t ld_stream;
+} dspark_verify_layer;
+
+int dspark_verify_step(const dspark_verify_args* args, const dspark_verify_layer* layers, int64_t count,
+                       dspark_stream stream);
+
 /* out[m] = argmax over V of logits[m] (bf16; first index of the maximum). Replaces
  * mx.argmax(v_logits[0], -1) of the verify loop (generate.py:1548). */
 int dspark_argmax_rows(const void* logits, int64_t ld, int64_t M, int64_t V, int32_t* out, dspark_stream stream);

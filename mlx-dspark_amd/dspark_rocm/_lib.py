@@ -76,6 +76,18 @@ class QmmPackedProblem(ctypes.Structure):
     ]
 
 
+class VerifyArgs(ctypes.Structure):
+    """dspark_verify_args (include/dspark.h)."""
+    _fields_ = ([(n, c_i64) for n in ("M", "H", "I", "Hq", "Hk", "D", "pos0", "kv_bits")]
+                + [(n, ctypes.c_double) for n in ("eps", "rope_base", "scale")]
+                + [(n, c_void_p) for n in ("h", "y", "r", "q", "k", "v", "qatt", "att", "hm", "qmm_ws")]
+                + [("qmm_ws_bytes", c_i64), ("attn_ws", c_void_p), ("attn_ws_bytes", c_i64),
+                   ("final_norm", c_void_p), ("head", c_void_p), ("head_bits", c_i64), ("vocab", c_i64),
+                   ("logits", c_void_p)])
+
+
+VERIFY_LAYER_FIELDS = 30   # 8-byte fields of dspark_verify_layer
+
 MAX_QMM_PROBLEMS = 4
 
 # name -> (restype, argtypes). Every symbol include/dspark.h declares.
@@ -165,6 +177,7 @@ SIGNATURES: dict[str, tuple] = {
                                                  c_void_p, c_void_p, c_void_p, c_i64_p, c_i64_p, c_int, c_int,
                                                  c_void_p]),
     "dspark_swiglu": (c_int, [c_void_p, c_i64, c_void_p, c_i64, c_i64, c_i64, c_void_p, c_i64, c_void_p]),
+    "dspark_verify_step": (c_int, [ctypes.POINTER(VerifyArgs), c_void_p, c_i64, c_void_p]),
     "dspark_argmax_rows": (c_int, [c_void_p, c_i64, c_i64, c_i64, c_void_p, c_void_p]),
     "dspark_greedy_accept": (c_int, [c_void_p, c_i64, c_void_p, c_void_p, c_void_p]),
     "dspark_argmax_accept_workspace": (c_size_t, [c_i64, c_i64]),

@@ -26,13 +26,14 @@ the greedy round (generate.py:1544-1593).
 
 from __future__ import annotations
 
+import ctypes
 import math
 from dataclasses import dataclass
 
 import torch
 from torch import nn
 
-from . import fast, ops
+from . import _lib, fast, ops
 from ._lib import load as _lib_load
 from .kv_cache import KVCache, QuantizedKVCache
 from .nn import QuantizedLinear
@@ -308,6 +309,7 @@ class VerifyEngine:
         self.n_acc = torch.zeros(1, dtype=torch.int32, device=dev)
         # The engine's own workspaces, sized once for every launch of a step at up to max_rows
         # rows and any cache length, so a captured step never sees them move.
+        self._widths = (hq * d, hk * d, hk * d, H, I, H)     # outputs of q, k, v, o, gate / up, down
         self.qmm_ws = ops.new_qmm_workspace(dev, self._qmm_workspace_need())
         self.accept_ws = torch.zeros(max(ops.argmax_accept_workspace_bytes(max_rows, a.vocab_size), 256),
                                      dtype=torch.uint8, device=dev)
@@ -317,6 +319,67 @@ class VerifyEngine:
         self.fused = e(max_rows, 0)
         self.attn_ws = torch.empty(max(ops.attention_workspace_bound(1, hq, hk, d, max_rows), 16), dtype=torch.uint8,
                                    device=dev)
+
+    def _native_layers(self, M: int, cache: list, pos0: int) -> list[int] | None:
+        """The layers of this step as ``dspark_verify_step`` takes them (the 8-byte fields of
+        ``dspark_verify_layer``, in order), or None when some projection is not packed or a cache is
+        not one of the module's own in bf16: those steps are enqueued launch by launch. Built from
+        the modules and caches as they are now; nothing is kept."""
+        a = self.args
+        kv_bits = getattr(cache[0], "bits", 0)
+        kind = QuantizedKVCache if kv_bits else KVCache
+        H = a.hidden_size
+        row = self.h.data_ptr()
+        slot = {li: j for j, li in enumerate(self.tap)}
+        fused, ld = self.fused.data_ptr(), self.fused.shape[1]
+        pk, out = self._packed, []
+        for li, (layer, c) in enumerate(zip(self.model.layers, cache)):
+            at, mlp = layer.self_attn, layer.mlp
+            packs = [pk.get(id(mod)) for mod in (at.q_proj, at.k_proj, at.v_proj, at.o_proj)]
+            packs += [self._swiglu.get(id(mlp)), pk.get(id(mlp.down_proj))]
+            if None in packs or type(c) is not kind or c.dtype != torch.bfloat16 or c.capacity < pos0 + M:
+                return None
+            q, k, v, o, pair, down = packs
+            if not q.bits == k.bits == v.bits or (q.n, k.n, v.n, o.n, pair.n, down.n) != self._widths \
+                    or (q.k, k.k, v.k, pair.k, o.k, down.k) != (H, H, H, H, q.n, pair.n):
+                return None
+            out += [t.data_ptr() for t in (layer.input_layernorm, at.q_norm, at.k_norm, layer.post_attention_layernorm)]
+            out += [p.buf.data_ptr() for p in packs]
+            out += [q.bits, o.bits, pair.bits, down.bits]
+            if kv_bits:
+                (kw, ks, kb), (vw, vs, vb) = c.keys, c.values
+                if c.bits != kv_bits or c.group_size != 64 or ks.stride() != kb.stride() or vs.stride() != vb.stride():
+                    return None
+                out += [kw.data_ptr(), vw.data_ptr(), *kw.stride()[1:3], *vw.stride()[1:3]]
+                out += [t.data_ptr() for t in (ks, kb, vs, vb)]
+                out += [*ks.stride()[1:3], *vs.stride()[1:3]]
+            else:
+                kw, vw = c.keys, c.values
+                out += [kw.data_ptr(), vw.data_ptr(), *kw.stride()[1:3], *vw.stride()[1:3]] + [0] * 8
+            j = slot.get(li)
+            out += [row, H] if j is None else [fused + 2 * j * H, ld]
+        return out
+
+    def _native_step(self, M: int, cache: list, pos0: int) -> bool:
+        """The step's launches after the embedding, from native code; False when they are the
+        caller's to make (:meth:`_native_layers`)."""
+        a, m = self.args, self.model
+        head = self._packed.get(id(m.lm_head))
+        if head is None or (head.n, head.k) != (a.vocab_size, a.hidden_size) or len(cache) != len(m.layers):
+            return False
+        layers = self._native_layers(M, cache, pos0)
+        if not layers:
+            return False
+        assert len(layers) == _lib.VERIFY_LAYER_FIELDS * len(m.layers)
+        bufs = (self.h, self.y, self.r, self.q, self.k, self.v, self.qatt, self.att, self.hm, self.qmm_ws)
+        args = _lib.VerifyArgs(M, a.hidden_size, a.intermediate_size, a.num_attention_heads, a.num_key_value_heads,
+                               a.head_dim, pos0, getattr(cache[0], "bits", 0), a.rms_norm_eps, a.rope_theta,
+                               a.head_dim ** -0.5, *(t.data_ptr() for t in bufs), self.qmm_ws.numel(),
+                               self.attn_ws.data_ptr(), self.attn_ws.numel(), m.norm.data_ptr(), head.buf.data_ptr(),
+                               head.bits, a.vocab_size, self.logits.data_ptr())
+        _lib.call("dspark_verify_step", args, (ctypes.c_int64 * len(layers))(*layers), len(m.layers),
+                  torch.cuda.current_stream(self.h.device).cuda_stream)
+        return True
 
     def _qmm_workspace_need(self) -> int:
         a, m, M = self.args, self.model, self.max_rows
@@ -363,10 +426,19 @@ class VerifyEngine:
         tokens ``self.tt[:M]`` and the accepted count ``self.n_acc`` for ``self.draft[:M-1]``;
         the tapped layers' residual streams (``set_tap``) in ``self.fused[:M]``.
         Enqueues kernels only (graph-capturable for a fixed pos0)."""
+        torch.index_select(self.model.embed_tokens, 0, self.ids[:M], out=self.h[:M])
+        logits = self.logits[:M]
+        if not self._native_step(M, cache, pos0):
+            self._launch_step(M, cache, pos0)
+        if accept:
+            ops.argmax_accept(logits, self.draft[:M - 1], self.tt[:M], self.n_acc, self.accept_ws)
+        return logits
+
+    def _launch_step(self, M: int, cache: list[KVCache], pos0: int) -> None:
+        """The step's launches after the embedding, one by one."""
         a, m = self.args, self.model
         hq, hk, d, eps = a.num_attention_heads, a.num_key_value_heads, a.head_dim, a.rms_norm_eps
         h, r, y = self.h[:M], self.r[:M], self.y[:M]
-        torch.index_select(m.embed_tokens, 0, self.ids[:M], out=h)
         L = pos0 + M
         H = a.hidden_size
         slot = {li: j for j, li in enumerate(self.tap)}
@@ -419,12 +491,7 @@ class VerifyEngine:
                 ops.swiglu(self.g[:M], self.u[:M], out=self.hm[:M])
             self._qmm(self.hm[:M], [mlp.down_proj], [r])
         ops.rmsnorm(hcur, m.norm, eps, residual=r, h_out=stream_out(len(m.layers) - 1), out=y)
-        lm = m.lm_head
-        logits = self.logits[:M]
-        self._qmm(y, [lm], [logits])
-        if accept:
-            ops.argmax_accept(logits, self.draft[:M - 1], self.tt[:M], self.n_acc, self.accept_ws)
-        return logits
+        self._qmm(y, [m.lm_head], [self.logits[:M]])
 
 
 class Target:
