@@ -137,9 +137,19 @@ inline Plan make_plan(long B, long Hq, long Hk, long Mq, long D, long L) {
   const long heads = B * Hk * p.NRG;
   const long target = (p.WV == 8 || D == 256) ? 256 : 512;
   long nb = (target + heads - 1) / heads;
-  const long min_keys = L <= 1280 ? 64 : (L < 4096 ? 128 : 256);
+  // Head dim 256 keeps 128 keys (four of its tiles) beyond that, where few KV heads otherwise leave
+  // half the CUs idle: 24/4 heads, 6 rows, 10007 keys 29.9 -> 26.9 us over an 8-bit cache, 20.3 ->
+  // 18.7 over bf16; 16 rows 53.7 -> 45.6 and 27.0 -> 25.0; but over 5000 keys 16 rows (more than 4
+  // row tiles) lose more to the partials than they gain (8-bit 31.4 -> 36.6).
+  const bool short_blocks = L < 4096 || (D == 256 && (p.RT <= 4 || L >= 8192));
+  const long min_keys = L <= 1280 ? 64 : (short_blocks ? 128 : 256);
   const long max_nb = (L + min_keys - 1) / min_keys;
   if (nb > max_nb) nb = max_nb;
+  // Somewhat more than one workgroup a CU leaves most CUs waiting for those with two: one each
+  // instead (32/8 heads x 128, 16 rows: 8500 keys 19.3 -> 16.8 us, 10007 keys 20.3 -> 17.6, over an
+  // 8-bit cache 27.2 -> 23.1). Not beyond one and a half (14000 keys, 6 rows, 8-bit: 22.0 -> 22.9),
+  // nor for the single row tile of a plain decode step (12000 keys: 17.1 -> 19.1).
+  if (D <= 128 && target == 512 && p.RT > 1 && heads * nb > 256 && heads * nb <= 384) nb = (256 + heads - 1) / heads;
   if (nb < 1) nb = 1;
   if (p.WV == 4 && D <= 128 && heads * nb < 256) p.KS = 2;
   long chunk = (L + nb - 1) / nb;
