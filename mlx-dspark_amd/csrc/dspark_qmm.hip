@@ -84,14 +84,17 @@ Plan make_plan(const long* Ns, int count, long K, long M, int bits, bool wholek_
   }
   // 16 groups (1024 k) per slice, unless those workgroups fill their last resident round
   // (one or two rounds) poorly and 8-group slices, whose kernels keep more workgroups per CU,
-  // fill theirs better. Resident workgroups per CU of the instantiations (VGPR-limited, as
+  // fill theirs better (and are not cut back by the slice limit: 34 slices of K = 17408 became 32
+  // uneven ones through the 16-group kernel, [5120, 17408] 4-bit 23.3 us against 19.7 in 17). Resident workgroups per CU of the instantiations (VGPR-limited, as
   // compiled): 16-group 3 (8-bit) / 4 (4-bit), 8-group 5.
   long s = (G + 15) / 16;
   {
     auto fill = [&](long w, long slots) { return (double)w / (double)(((w + slots - 1) / slots) * slots); };
     const long slots16 = kCUs * (bits == 8 ? 3 : 4), slots8 = kCUs * 5;
     const long w16 = strips * s, s8 = (G + 7) / 8;
-    if (w16 <= 2 * slots16 && fill(w16, slots16) < 0.9 && fill(strips * s8, slots8) > fill(w16, slots16)) s = s8;
+    if (s8 <= kQmmMaxSlices && w16 <= 2 * slots16 && fill(w16, slots16) < 0.9 &&
+        fill(strips * s8, slots8) > fill(w16, slots16))
+      s = s8;
   }
   if (s > kQmmMaxSlices) s = kQmmMaxSlices;
   if (s > max_slices(G, bits)) s = max_slices(G, bits);
