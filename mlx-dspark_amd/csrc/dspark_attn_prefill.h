@@ -19,7 +19,6 @@
 //   * K and V tiles are copied global -> LDS without passing registers, double buffered, one
 //     barrier a tile; 16-byte chunks XOR-swizzled by the row, so both kinds of read are free of
 //     bank conflicts;
-//   * two workgroups share a CU: one's softmax runs under the other's MFMAs;
 //   * a grid of fewer than two workgroups a CU splits the keys (fp32 partials and a combine);
 //   * the row tiles of one KV head are consecutive on one XCD, whose L2 then holds its K and V;
 //     long causal tiles first.
@@ -39,8 +38,7 @@ constexpr int kThreads = 256;
 constexpr int kRows = 128;  // query rows of a workgroup
 constexpr float kLowest = -3.402823466e38f;
 
-template <int D>
-constexpr int kKeys = D == 256 ? 32 : 64;  // keys of a tile
+constexpr int kKeys = 64;   // keys of a tile
 
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
@@ -111,9 +109,12 @@ __device__ __forceinline__ void split(const f32x16_t& p, int r0, u32x4_t (&o)[kP
   }
 }
 
+// Head dim 256 takes one workgroup a CU: its queries and outputs alone are 192 registers, and two
+// workgroups spilled 33 over 32-key tiles (24/4 heads, 2048 rows, bf16 218 us, fp16 205; so 200 and
+// 154; 16/8 heads, 1500 rows over 3000 keys 196 -> 178 and 178 -> 152).
 template <class T, int D>
-__global__ __launch_bounds__(kThreads, 2) void prefill_kernel(const Args a) {
-  constexpr int KT = kKeys<D>, SUB = KT / 32, CH = D / 8, NJ = KT * CH / kThreads, ND = D / 32, NK = D / 16;
+__global__ __launch_bounds__(kThreads, D == 256 ? 1 : 2) void prefill_kernel(const Args a) {
+  constexpr int KT = kKeys, SUB = KT / 32, CH = D / 8, NJ = KT * CH / kThreads, ND = D / 32, NK = D / 16;
   constexpr int NP = kPieces<T>;
   __shared__ __attribute__((aligned(16))) u16 sm[2][2][KT * D];  // [buffer][K, V]
   typedef __attribute__((address_space(3))) u16 lds_u16;
@@ -237,6 +238,9 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_kernel(const Args a) {
       }
     }
     l += sum;
+    // Head dim 64, where the products are the shorter phase: ahead of the other workgroup's softmax
+    // (2000 rows over 4000 keys 53 -> 46 us, 2048 over 2048 32.6 -> 29.2; at 128 a first chunk lost 9%)
+    if constexpr (D == 64) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int u = 0; u < SUB; ++u)
 #pragma unroll
@@ -259,6 +263,7 @@ __global__ __launch_bounds__(kThreads, 2) void prefill_kernel(const Args a) {
             for (int d = 0; d < DB; ++d) o[d0 + d] = mfma32<T>(vf[d], p[n], o[d0 + d]);
         }
       }
+    if constexpr (D == 64) __builtin_amdgcn_s_setprio(0);
   }
 
   l += shfl_xor(l, 32);

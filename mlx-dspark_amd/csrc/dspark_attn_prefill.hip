@@ -13,15 +13,13 @@ struct Plan {
   size_t part_floats;
 };
 
-inline long tile_keys(long D) { return D == 256 ? 32 : 64; }
-
 Plan make_plan(long B, long Hq, long Hk, long M, long L, long D) {
   Plan p{};
   const long R = Hq / Hk * M;
   p.tiles = (int)((R + kRows - 1) / kRows);
   const long blocks = B * Hk * p.tiles;
   // Key splits up to two workgroups per CU, of at least four tiles each
-  const long s = std::min((512 + blocks / 2) / blocks, (L + 4 * tile_keys(D) - 1) / (4 * tile_keys(D)));
+  const long s = std::min((512 + blocks / 2) / blocks, (L + 4 * kKeys - 1) / (4 * kKeys));
   p.S = (int)std::max(1L, s);
   p.part_floats = p.S > 1 ? (size_t)p.S * B * Hk * R * (D + 2) : 0;
   return p;

@@ -5,7 +5,7 @@ the errors of the fp32 path: a score is off by at most (D + 2) units of 2^-24 of
 and its exponent's argument by as much again of its size, a probability by that and the unit 2^-22 of
 its pieces, the two sums over L keys by L / 16 units (16 keys a lane are added in turn, 16 or more in
 the matrix core); numerator and denominator both, over sum p |v|.
-Sizes sit at the edges of the 32-row waves, 128-row workgroups, 32 / 64-key tiles and key splits.
+Sizes sit at the edges of the 32-row waves, 128-row workgroups, 64-key tiles and key splits.
 """
 
 from __future__ import annotations
