@@ -19,7 +19,7 @@
 //   * K and V tiles are copied global -> LDS without passing registers, double buffered, one
 //     barrier a tile; 16-byte chunks XOR-swizzled by the row, so both kinds of read are free of
 //     bank conflicts;
-//   * a grid of fewer than two workgroups a CU splits the keys (fp32 partials and a combine);
+//   * a grid that would leave CUs idle for long splits the keys (fp32 partials and a combine);
 //   * the row tiles of one KV head are consecutive on one XCD, whose L2 then holds its K and V;
 //     long causal tiles first.
 // Measured: 2048 rows behind 2953 keys, 32/8 heads x 128, bf16: 252 us (528 TFLOP/s of the two

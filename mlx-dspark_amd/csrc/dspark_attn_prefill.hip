@@ -18,9 +18,25 @@ Plan make_plan(long B, long Hq, long Hk, long M, long L, long D) {
   const long R = Hq / Hk * M;
   p.tiles = (int)((R + kRows - 1) / kRows);
   const long blocks = B * Hk * p.tiles;
-  // Key splits up to two workgroups per CU, of at least four tiles each
-  const long s = std::min((512 + blocks / 2) / blocks, (L + 4 * kKeys - 1) / (4 * kKeys));
-  p.S = (int)std::max(1L, s);
+  // Key splits by a model of the call's time in us, fitted to sweeps of 1 to 16 splits (17 to 2048 rows,
+  // 400 to 4096 keys, 8 to 376 blocks; within 15% of the best split everywhere): W workgroups a CU
+  // take their key tiles in turn, a lone one (whose longest causal tile counts) at a slower pace;
+  // splits cost the combine's launch and their partials, written and read at 4.1 TB/s. 32/8 heads x
+  // 128: 777 rows and keys 30.8 us in one split, 37.8 in three; 300 rows over 3000 keys 91 and 49;
+  // 100 over 4000 keys 34.8 in 8, 38.2 in 16; 64/8, 400 rows and keys 20.4 in one, 33.5 in three.
+  const double lone = D == 256 ? 3.6 : D == 128 ? 1.76 : 1.43, shared = D == 256 ? 3.6 : D == 128 ? 1.27 : 0.96;
+  const long longest = (L + kKeys - 1) / kKeys;
+  const double mean = (L - 0.5 * std::min(M, L)) / kKeys, rows = (double)B * Hq * M;
+  double best = 0;
+  for (long s = 1; s <= std::min(64L, (longest + 3) / 4); ++s) {
+    const long w = (blocks * s + 255) / 256;
+    const double tiles = w == 1 ? (double)((longest + s - 1) / s) : std::max(1.0, mean / s);
+    const double cost = w * tiles * (w == 1 ? lone : shared) + (s > 1 ? 6 + s * rows * D * 8 / 4.1e6 : 0);
+    if (s == 1 || cost < best) {
+      best = cost;
+      p.S = (int)s;
+    }
+  }
   p.part_floats = p.S > 1 ? (size_t)p.S * B * Hk * R * (D + 2) : 0;
   return p;
 }
