@@ -22,6 +22,9 @@
 //   * a grid that would leave CUs idle for long splits the keys (fp32 partials and a combine);
 //   * the row tiles of one KV head are consecutive on one XCD, whose L2 then holds its K and V;
 //     long causal tiles first.
+// Tiles that hold no key a row sees are not read for it, so a value that is not finite there leaves
+// it alone; within the last tiles such a value times the zero probability is a NaN, as it is anywhere
+// in a product over all keys.
 // Measured: 2048 rows behind 2953 keys, 32/8 heads x 128, bf16: 252 us (528 TFLOP/s of the two
 // products, 1060 with the pieces) where torch's fp32 scores, softmax and product took 4042 us.
 #pragma once
