@@ -371,10 +371,12 @@ class VerifyEngine:
         if not layers:
             return False
         assert len(layers) == _lib.VERIFY_LAYER_FIELDS * len(m.layers)
-        bufs = (self.h, self.y, self.r, self.q, self.k, self.v, self.qatt, self.att, self.hm, self.qmm_ws)
+        bufs = (self.h, self.y, self.r, self.q, self.k, self.v, self.qatt, self.att, self.hm)
+        ws = self.qmm_ws                    # None when no product of the model splits K
         args = _lib.VerifyArgs(M, a.hidden_size, a.intermediate_size, a.num_attention_heads, a.num_key_value_heads,
                                a.head_dim, pos0, getattr(cache[0], "bits", 0), a.rms_norm_eps, a.rope_theta,
-                               a.head_dim ** -0.5, *(t.data_ptr() for t in bufs), self.qmm_ws.numel(),
+                               a.head_dim ** -0.5, *(t.data_ptr() for t in bufs),
+                               None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(),
                                self.attn_ws.data_ptr(), self.attn_ws.numel(), m.norm.data_ptr(), head.buf.data_ptr(),
                                head.bits, a.vocab_size, self.logits.data_ptr())
         _lib.call("dspark_verify_step", args, (ctypes.c_int64 * len(layers))(*layers), len(m.layers),

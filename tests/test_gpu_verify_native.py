@@ -67,3 +67,16 @@ def test_steps_it_leaves_alone(dev):
     assert torch.equal(tgt.verify(ids, other)[0], want)
     with pytest.raises(ValueError):
         tgt.engine.step(4, cache, cache[0].capacity)
+
+
+def test_step_without_a_qmm_workspace(dev, monkeypatch):
+    """A target whose matrices are all one K slice holds no qmm workspace; its steps are native too."""
+    from dspark_rocm.model import DenseModel, ModelArgs, Target, VerifyEngine
+
+    args = ModelArgs(hidden_size=512, num_hidden_layers=2, intermediate_size=512, num_attention_heads=4,
+                     num_key_value_heads=2, head_dim=128, vocab_size=1000, bits=8)
+    tgt = Target(DenseModel.random(args, device=dev, seed=3))
+    assert tgt.engine.qmm_ws is None and tgt.engine._native_layers(4, tgt.make_cache(8), 0)
+    got = _rounds(tgt, None)
+    monkeypatch.setattr(VerifyEngine, "_native_step", lambda self, *a: False)
+    assert all(torch.equal(g, w) for g, w in zip(got, _rounds(tgt, None)))
