@@ -320,11 +320,32 @@ class VerifyEngine:
         self.attn_ws = torch.empty(max(ops.attention_workspace_bound(1, hq, hk, d, max_rows), 16), dtype=torch.uint8,
                                    device=dev)
 
+    def _norm_fits(self, w: torch.Tensor, n: int) -> bool:
+        """Whether ``w`` is a norm weight the native step may pass as a bare pointer."""
+        return w.device == self.h.device and w.dtype == torch.bfloat16 and w.shape == (n,) and w.is_contiguous()
+
+    def _cache_fits(self, c, bits: int, need: int) -> bool:
+        """Whether every tensor of cache ``c`` holds ``need`` rows of the model's KV heads, batch 1, on
+        the engine's device, in the type and width its kernels read: the native step passes pointers
+        and strides, and the model's sizes for the rest."""
+        a, bf = self.args, torch.bfloat16
+        if bits:
+            if c.bits != bits or c.group_size != 64:
+                return False
+            forms = ((torch.int32, a.head_dim * bits // 32), (bf, a.head_dim // 64), (bf, a.head_dim // 64))
+            parts = [(t, *f) for trip in (c.keys, c.values) for t, f in zip(trip, forms)]
+        else:
+            parts = [(t, bf, a.head_dim) for t in (c.keys, c.values)]
+        return all(t.device == self.h.device and t.dtype == dt and t.dim() == 4 and t.shape[2] >= need
+                   and t.shape == (1, a.num_key_value_heads, t.shape[2], width) and t.stride(3) == 1
+                   for t, dt, width in parts)
+
     def _native_layers(self, M: int, cache: list, pos0: int) -> list[int] | None:
         """The layers of this step as ``dspark_verify_step`` takes them (the 8-byte fields of
-        ``dspark_verify_layer``, in order), or None when some projection is not packed or a cache is
-        not one of the module's own in bf16: those steps are enqueued launch by launch. Built from
-        the modules and caches as they are now; nothing is kept."""
+        ``dspark_verify_layer``, in order), or None when some projection is not packed, a cache is
+        not one of the module's own in bf16 or a tensor is not what its kernel will take it for:
+        those steps are enqueued launch by launch, with the checks (and refusals) of the single
+        launches. Built from the modules and caches as they are now; nothing is kept."""
         a = self.args
         kv_bits = getattr(cache[0], "bits", 0)
         kind = QuantizedKVCache if kv_bits else KVCache
@@ -337,7 +358,10 @@ class VerifyEngine:
             at, mlp = layer.self_attn, layer.mlp
             packs = [pk.get(id(mod)) for mod in (at.q_proj, at.k_proj, at.v_proj, at.o_proj)]
             packs += [self._swiglu.get(id(mlp)), pk.get(id(mlp.down_proj))]
-            if None in packs or type(c) is not kind or c.dtype != torch.bfloat16 or c.capacity < pos0 + M:
+            if None in packs or type(c) is not kind or not self._cache_fits(c, kv_bits, pos0 + M):
+                return None
+            if not (self._norm_fits(layer.input_layernorm, H) and self._norm_fits(layer.post_attention_layernorm, H)
+                    and self._norm_fits(at.q_norm, a.head_dim) and self._norm_fits(at.k_norm, a.head_dim)):
                 return None
             q, k, v, o, pair, down = packs
             if not q.bits == k.bits == v.bits or (q.n, k.n, v.n, o.n, pair.n, down.n) != self._widths \
@@ -348,7 +372,7 @@ class VerifyEngine:
             out += [q.bits, o.bits, pair.bits, down.bits]
             if kv_bits:
                 (kw, ks, kb), (vw, vs, vb) = c.keys, c.values
-                if c.bits != kv_bits or c.group_size != 64 or ks.stride() != kb.stride() or vs.stride() != vb.stride():
+                if ks.stride() != kb.stride() or vs.stride() != vb.stride():
                     return None
                 out += [kw.data_ptr(), vw.data_ptr(), *kw.stride()[1:3], *vw.stride()[1:3]]
                 out += [t.data_ptr() for t in (ks, kb, vs, vb)]
@@ -366,6 +390,8 @@ class VerifyEngine:
         a, m = self.args, self.model
         head = self._packed.get(id(m.lm_head))
         if head is None or (head.n, head.k) != (a.vocab_size, a.hidden_size) or len(cache) != len(m.layers):
+            return False
+        if not cache or not self._norm_fits(m.norm, a.hidden_size):
             return False
         layers = self._native_layers(M, cache, pos0)
         if not layers:

@@ -769,6 +769,9 @@ def qk_norm_rope_kv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_norm_w:
     M = q.shape[0]
     if k_cache.shape[1] < pos0 + M or v_cache.shape[1] < pos0 + M:
         raise ValueError(f"cache capacity {k_cache.shape[1]} < pos0 + M = {pos0 + M}")
+    for name, t in (("k_cache", k_cache), ("v_cache", v_cache)):
+        if t.dim() != 3 or t.shape[0] < kv_heads or t.shape[2] < head_dim:
+            raise ValueError(f"{name}: expected [{kv_heads}, capacity, {head_dim}], got {tuple(t.shape)}")
     ks = (ctypes.c_int64 * 2)(k_cache.stride(0), k_cache.stride(1))
     vs = (ctypes.c_int64 * 2)(v_cache.stride(0), v_cache.stride(1))
     _lib.call("dspark_qk_norm_rope_kv", _ptr(q), q.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), M, heads,
@@ -791,9 +794,13 @@ def qk_norm_rope_kv_quantized(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     for t in (ks, kb, vs, vb):
         _require_bf16("cache scales / biases", t)
     M = q.shape[0]
-    for name, t in (("key words", kw), ("value words", vw), ("key scales", ks), ("value scales", vs)):
+    W, G = head_dim * bits // 32, head_dim // group_size
+    for name, t, last in (("key words", kw, W), ("value words", vw, W), ("key scales", ks, G), ("key biases", kb, G),
+                          ("value scales", vs, G), ("value biases", vb, G)):
         if t.dim() != 3 or t.shape[1] < pos0 + M or t.stride(-1) != 1:
             raise ValueError(f"{name}: expected [Hk, capacity >= {pos0 + M}, ...] with unit last stride")
+        if t.shape[0] < kv_heads or t.shape[2] < last:
+            raise ValueError(f"{name}: expected [{kv_heads}, capacity, {last}], got {tuple(t.shape)}")
     if ks.stride() != kb.stride() or vs.stride() != vb.stride():
         raise ValueError("scales and biases of one cache must share strides")
     two = lambda t: (ctypes.c_int64 * 2)(t.stride(0), t.stride(1))
