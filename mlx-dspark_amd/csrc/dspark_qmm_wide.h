@@ -204,6 +204,10 @@ __device__ __forceinline__ void tile_loop(const Tile<MT, NT>& t, Smem<MT, NT>& s
     }
   }
 
+  // The requests above are the compiler's to order, so no count of later ones says that the first x
+  // tile has landed: all of them are waited for, once. In the loop the count holds, since the memory
+  // clobbers at a step's barrier keep its requests behind those of the steps before.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   if (tid < 64 * NT) *reinterpret_cast<u32x4_t*>(&sm.sc[(t.gs >> 3) & 1][tid * 8]) = scn;
   const int abase = c16 * 64 + ((k_chunk<BITS>(q) ^ ((c16 >> 1) & 7)) << 3);  // the second chunk: ^ 8
   const int sbase = (wave * 16 * NT + c16) * 8;
