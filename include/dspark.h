@@ -333,7 +333,8 @@ int dspark_verify_attention_typed(int dtype, const void* q, int64_t B, int64_t H
 /*
  * Attention over many query rows (prefill widths): out = softmax(scale * q . k^T) . v, causal (row
  * i sees keys 0 .. L - M + i) or over all L keys. fp32 scores, softmax and sums; the probabilities
- * keep their fp32 precision into the second product. q [B, Hq, M, D], K/V [B, Hk, L, D] of dtype
+ * keep their fp32 value into the second product (fp16: from 2^-28 of a row's largest on, and
+ * within 2^-51 of it below). q [B, Hq, M, D], K/V [B, Hk, L, D] of dtype
  * DSPARK_DTYPE_BF16 or _F16 through element strides {batch, head, position} (each a multiple of
  * 8, positions at most 2^22 elements apart; the last dim contiguous; all 16-byte aligned), D in {64, 128,
  * 256}, out a contiguous [B, Hq, M, D]. scale > 0; causal needs L >= M. Workspace 16-byte aligned,

@@ -2,9 +2,12 @@
 //
 // out[h, i] = softmax(scale * q[h, i] . k^T) . v with fp32 scores, softmax and sums, causal (row i
 // sees keys 0 .. L - M + i) or over all keys. q, k and v are bf16 or fp16, so every product of
-// q . k^T is exact; the probabilities keep fp32 precision into the second product: they go to the
-// matrix cores as kPieces pieces of the input type whose sum is the fp32 value (bf16: 3 x 8 bits;
-// fp16: 2 x 11 bits of p * 2^15, which keeps the pieces clear of the subnormals).
+// q . k^T is exact; the probabilities go to the matrix cores as kPieces pieces of the input type
+// whose sum is their fp32 value. bf16 pieces (8 bits each) have fp32's exponents. The fp16 ones
+// (11 bits) are of p * 2^15, the largest that fits, and the second and third, which lie below the
+// unit of the first, are scaled by another kLow = 2^12 and summed apart within a tile: the pieces are
+// exact from p = 2^-28 of the row's largest on, and below that less than 2^-51 of it short. (With two
+// pieces in one sum p = 2^-26 was 2^-14 off, and a quarter of all p 2^-23.)
 //
 // What bounds it: the MFMA pipe (at D = 128, per 32 queries x 64 keys 512 cycles of q . k^T and
 // 512 kPieces of p . v) and beside it the VALU (about 10 instructions a score, the exponential at
@@ -87,23 +90,32 @@ __device__ __forceinline__ u32x2_t lds_tr(const u16* p) {
   return __builtin_bit_cast(u32x2_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p));
 }
 
-template <class T>
-constexpr int kPieces = T::kF16 ? 2 : 3;
+constexpr int kPieces = 3;        // of a probability
+constexpr float kLow = 4096.f;    // the scale of fp16's second and third
 
-// Eight probabilities as pieces of the input type
+// Eight probabilities as pieces of the input type. fp16 rounds toward zero (two values an
+// instruction), which leaves 13 and then 2 of the 24 bits.
 template <class T>
-__device__ __forceinline__ void split(const f32x16_t& p, int r0, u32x4_t (&o)[kPieces<T>]) {
+__device__ __forceinline__ void split(const f32x16_t& p, int r0, u32x4_t (&o)[kPieces]) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     float a = p[r0 + 2 * i], b = p[r0 + 2 * i + 1];
 #pragma unroll
-    for (int n = 0; n < kPieces<T>; ++n) {
-      o[n][i] = attn::pack2<T>(a, b);
-      if (n + 1 < kPieces<T>) {
-        if constexpr (T::kF16) {
-          a -= attn::to_f32<T>(o[n][i] & 0xFFFFu);
-          b -= attn::to_f32<T>(o[n][i] >> 16);
-        } else {
+    for (int n = 0; n < kPieces; ++n) {
+      if constexpr (T::kF16) {
+        const attn::f16x2_t h = __builtin_bit_cast(attn::f16x2_t, __builtin_amdgcn_cvt_pkrtz(a, b));
+        o[n][i] = __builtin_bit_cast(u32, h);
+        if (n == 0) {
+          a = __builtin_fmaf((float)h.x, -kLow, a * kLow);
+          b = __builtin_fmaf((float)h.y, -kLow, b * kLow);
+        } else if (n == 1) {
+          const float m1 = __builtin_bit_cast(float, opaque_sgpr(0xBF800000u));  // keeps it one v_fma_mix
+          a = __builtin_fmaf((float)h.x, m1, a);
+          b = __builtin_fmaf((float)h.y, m1, b);
+        }
+      } else {
+        o[n][i] = attn::pack2<T>(a, b);
+        if (n + 1 < kPieces) {
           a -= __builtin_bit_cast(float, o[n][i] << 16);
           b -= __builtin_bit_cast(float, o[n][i] & 0xFFFF0000u);
         }
@@ -113,12 +125,11 @@ __device__ __forceinline__ void split(const f32x16_t& p, int r0, u32x4_t (&o)[kP
 }
 
 // Head dim 256 takes one workgroup a CU: its queries and outputs alone are 192 registers, and two
-// workgroups spilled 33 over 32-key tiles (24/4 heads, 2048 rows, bf16 218 us, fp16 205; so 200 and
-// 154; 16/8 heads, 1500 rows over 3000 keys 196 -> 178 and 178 -> 152).
+// workgroups spilled 33 over 32-key tiles (bf16, 24/4 heads, 2048 rows: 218 us, so 200; 16/8 heads,
+// 1500 rows over 3000 keys 196 -> 178).
 template <class T, int D>
 __global__ __launch_bounds__(kThreads, D == 256 ? 1 : 2) void prefill_kernel(const Args a) {
   constexpr int KT = kKeys, SUB = KT / 32, CH = D / 8, NJ = KT * CH / kThreads, ND = D / 32, NK = D / 16;
-  constexpr int NP = kPieces<T>;
   __shared__ __attribute__((aligned(16))) u16 sm[2][2][KT * D];  // [buffer][K, V]
   typedef __attribute__((address_space(3))) u16 lds_u16;
   typedef const __attribute__((address_space(1))) u16 glb_u16;
@@ -244,28 +255,60 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 1 : 2) void prefill_kernel(con
     // Head dim 64, where the products are the shorter phase: ahead of the other workgroup's softmax
     // (2000 rows over 4000 keys 53 -> 46 us, 2048 over 2048 32.6 -> 29.2; at 128 a first chunk lost 9%)
     if constexpr (D == 64) __builtin_amdgcn_s_setprio(1);
+    auto v_frag = [&](int uj, int d) {  // V^T of keys 16 uj .. 16 uj + 15, columns 32 d ..
+      const u16* vp = vs + 16 * uj * D + vbase + (((4 * d + vchunk) ^ vswz) << 3);
+      const u32x2_t lo = lds_tr(vp), hi = lds_tr(vp + 8 * D);
+      return u32x4_t{lo.x, lo.y, hi.x, hi.y};
+    };
+    if constexpr (T::kF16) {
+      // Two column blocks of scaled sums at a time: sums kept over the tiles (as many registers as the
+      // outputs) spilled at head dim 128 and moved 1346 registers a tile at 256. Against two pieces in
+      // one sum: 2048 rows over 5001 keys, 32/8 x 128, 226 -> 271 us; 24/4 x 256, 2048 rows, 155 -> 205.
+      constexpr int DB = 2;
+      u32x4_t p[2 * SUB][kPieces];
 #pragma unroll
-    for (int u = 0; u < SUB; ++u)
+      for (int d0 = 0; d0 < ND; d0 += DB) {
+        f32x16_t low[DB];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        u32x4_t p[NP];
-        split<T>(s[u], 8 * j, p);
-        constexpr int DB = ND < 4 ? ND : 4;  // V fragments in flight
+        for (int d = 0; d < DB; ++d)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) low[d][r] = 0.f;
+#pragma unroll
+        for (int uj = 0; uj < 2 * SUB; ++uj) {
+          if (d0 == 0) split<T>(s[uj >> 1], 8 * (uj & 1), p[uj]);
+          u32x4_t vf[DB];
+#pragma unroll
+          for (int d = 0; d < DB; ++d) vf[d] = v_frag(uj, d0 + d);
+#pragma unroll
+          for (int d = 0; d < DB; ++d) o[d0 + d] = mfma32<T>(vf[d], p[uj][0], o[d0 + d]);
+#pragma unroll
+          for (int n = 1; n < kPieces; ++n)
+#pragma unroll
+            for (int d = 0; d < DB; ++d) low[d] = mfma32<T>(vf[d], p[uj][n], low[d]);
+        }
+#pragma unroll
+        for (int d = 0; d < DB; ++d)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[d0 + d][r] = __builtin_fmaf(low[d][r], 1.f / kLow, o[d0 + d][r]);
+      }
+    } else {
+      constexpr int DB = ND < 4 ? ND : 4;  // V fragments in flight
+#pragma unroll
+      for (int uj = 0; uj < 2 * SUB; ++uj) {
+        u32x4_t p[kPieces];
+        split<T>(s[uj >> 1], 8 * (uj & 1), p);
 #pragma unroll
         for (int d0 = 0; d0 < ND; d0 += DB) {
           u32x4_t vf[DB];
 #pragma unroll
-          for (int d = 0; d < DB; ++d) {
-            const u16* vp = vs + (32 * u + 16 * j) * D + vbase + (((4 * (d0 + d) + vchunk) ^ vswz) << 3);
-            const u32x2_t lo = lds_tr(vp), hi = lds_tr(vp + 8 * D);
-            vf[d] = u32x4_t{lo.x, lo.y, hi.x, hi.y};
-          }
+          for (int d = 0; d < DB; ++d) vf[d] = v_frag(uj, d0 + d);
 #pragma unroll
-          for (int n = 0; n < NP; ++n)
+          for (int n = 0; n < kPieces; ++n)
 #pragma unroll
             for (int d = 0; d < DB; ++d) o[d0 + d] = mfma32<T>(vf[d], p[n], o[d0 + d]);
         }
       }
+    }
     if constexpr (D == 64) __builtin_amdgcn_s_setprio(0);
   }
 

@@ -2,8 +2,8 @@
 
 Against float64 attention of the same inputs. Bound per output: half a unit of the output type, plus
 the errors of the fp32 path: a score is off by at most (D + 2) units of 2^-24 of scale * sum |q k|
-and its exponent's argument by as much again of its size, a probability by that and the unit 2^-22 of
-its pieces, the two sums over L keys by L / 16 units (16 keys a lane are added in turn, 16 or more in
+and its exponent's argument by as much again of its size, a probability by that and the units of its
+exponential, the two sums over L keys by L / 16 units (16 keys a lane are added in turn, 16 or more in
 the matrix core); numerator and denominator both, over sum p |v|.
 Sizes sit at the edges of the 32-row waves, 128-row workgroups, 64-key tiles and key splits.
 """
@@ -142,3 +142,29 @@ def test_capture_replays_on_new_inputs(dev):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, run())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d,L", [(64, 33), (128, 90), (256, 90), (64, 1200), (128, 1200), (256, 1200)])
+def test_small_probabilities_keep_fp32_precision(dev, dtype, d, L):
+    """The largest weight of every row falls on a key whose value is zero, so probabilities of e^-gap
+    of it make up the output. All are equal, so what their pieces lose does not average out. The
+    scores are exact; the bound is half a unit of the output type, the fp32 errors of the exponent's
+    argument (3 units of its size, gap) and the units of the two sums."""
+    from dspark_rocm import fast
+
+    g = torch.Generator(device=dev).manual_seed(3)
+    for gap in (9.625, 13.25, 17.25, 18.875, 20.125, 22.75):
+        q = torch.zeros((1, 4, 24, d), dtype=dtype, device=dev)
+        q[..., 0] = 1
+        k = torch.zeros((1, 2, L, d), dtype=dtype, device=dev)
+        k[:, :, 5, 0] = gap
+        v = (torch.rand((1, 2, L, d), generator=g, device=dev) * 3e4 + 3e4).to(dtype)
+        v[:, :, 5] = 0
+        for mask in (None, "causal") if L > 33 else (None,):
+            assert fast.prefill_kernel(q, k, v, 1.0, mask, None)
+            out = fast.scaled_dot_product_attention(q, k, v, scale=1.0, mask=mask)
+            ref = _reference(q, k, v, 1.0, mask == "causal")[0]
+            bound = (UNIT[dtype] + (3 * gap + 8 + L / 16) * 2.0 ** -24) * ref.abs() + 2.0 ** -25
+            worst = float(((out.double() - ref).abs() / bound).max())
+            assert worst <= 1, f"gap {gap} {mask}: {worst} of the bound"
