@@ -27,7 +27,9 @@
 //     long causal tiles first.
 // Tiles that hold no key a row sees are not read for it, so a value that is not finite there leaves
 // it alone; within the last tiles such a value times the zero probability is a NaN, as it is anywhere
-// in a product over all keys.
+// in a product over all keys. Where a row does see it, the zero and negative pieces would make a NaN of
+// an infinity too, and values near the end of bf16's range overflow the unnormalised sum: outputs that
+// are not finite are looked at again (plain_row).
 // Measured: 2048 rows behind 2953 keys, 32/8 heads x 128, bf16: 252 us (528 TFLOP/s of the two
 // products, 1060 with the pieces) where torch's fp32 scores, softmax and product took 4042 us.
 #pragma once
@@ -122,6 +124,83 @@ __device__ __forceinline__ void split(const f32x16_t& p, int r0, u32x4_t (&o)[kP
       }
     }
   }
+}
+
+__device__ __forceinline__ bool not_finite(float v) { return !(__builtin_fabsf(v) < __builtin_inff()); }
+
+// The D / 64 adjacent columns of a lane
+template <int D>
+struct LaneCols {
+  u16 c[D / 64];
+};
+
+// One row (of KV head bh) that has outputs which are not finite, again, by one wave; m and l are its
+// maximum and denominator. Those of columns with such values among the row's keys are the sum of
+// these (a NaN, an infinity, or both infinities). Columns with such values only among the keys after
+// them that share its last tile (32 positions of a wave's rows, 64 keys) stay NaN. In the others the
+// unnormalised sum overflowed: they become the plain sum of fp32 probability times value. An infinite
+// value in the first key of 2048 rows over 5001, 32/8 heads x 128: 5.1 ms (the torch ops 4.1).
+template <class T, int D>
+__device__ __forceinline__ void plain_row(const Args& a, int bh, int row, float m, float l) {
+  constexpr int C = D / 64;
+  const int lane = threadIdx.x & 63, b = bh / a.Hk, hk = bh - b * a.Hk;
+  const int pos = row / a.gqa, hq = hk * a.gqa + (row - pos * a.gqa);
+  const int keys = a.causal ? a.L - a.M + pos + 1 : a.L;
+  const u16* v = a.v + b * a.vsb + hk * a.vsh + lane * C;
+  auto cols = [&](int key) { return *reinterpret_cast<const LaneCols<D>*>(v + key * a.vss); };
+  u16* op = a.out + (((long)b * a.Hk * a.gqa + hq) * a.M + pos) * D + lane * C;
+  float sum[C] = {}, after[C] = {};
+  auto add = [&](int key, float (&to)[C]) {
+    const LaneCols<D> x = cols(key);
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const float f = attn::to_f32<T>(x.c[c]);
+      to[c] += not_finite(f) ? f : 0.f;
+    }
+  };
+#pragma unroll 8
+  for (int k = 0; k < keys; ++k) add(k, sum);
+#pragma unroll 1
+  for (int k = keys; k < min(keys + 32 + kKeys, a.L); ++k) add(k, after);
+  bool over[C], any = false;
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const bool bad = not_finite(attn::to_f32<T>(op[c]));
+    over[c] = bad && !not_finite(sum[c]) && !not_finite(after[c]);
+    if (bad && not_finite(sum[c])) op[c] = attn::from_f32<T>(sum[c]);
+    any |= over[c];
+    sum[c] = 0.f;
+  }
+  if (!__builtin_amdgcn_ballot_w64(any)) return;
+  const u16* q = a.q + b * a.qsb + hq * a.qsh + pos * a.qss;
+  const u16* kr = a.k + b * a.ksb + hk * a.ksh;
+  const float inv = (T::kF16 ? 32768.f : 1.f) / l;
+#pragma unroll 1
+  for (int k0 = 0; k0 < keys; k0 += 64) {  // a lane takes a key's score
+    const int n = min(64, keys - k0);
+    const u16* kp = kr + (k0 + min(lane, n - 1)) * a.kss;
+    float s = 0.f;
+#pragma unroll 1
+    for (int c = 0; c < D; c += 8) {
+      const u32x4_t x = ldg128(q + c), y = ldg128(kp + c);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s = __builtin_fmaf(attn::to_f32<T>(x[i] & 0xFFFFu), attn::to_f32<T>(y[i] & 0xFFFFu), s);
+        s = __builtin_fmaf(attn::to_f32<T>(x[i] >> 16), attn::to_f32<T>(y[i] >> 16), s);
+      }
+    }
+    const float p = __builtin_amdgcn_exp2f((s - m) * a.scale_log2) * inv;
+#pragma unroll 1
+    for (int j = 0; j < n; ++j) {
+      const float pj = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, p), j));
+      const LaneCols<D> x = cols(k0 + j);
+#pragma unroll
+      for (int c = 0; c < C; ++c) sum[c] = __builtin_fmaf(pj, attn::to_f32<T>(x.c[c]), sum[c]);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+    if (over[c]) op[c] = attn::from_f32<T>(sum[c]);
 }
 
 // Head dim 256 takes one workgroup a CU: its queries and outputs alone are 192 registers, and two
@@ -313,8 +392,9 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 1 : 2) void prefill_kernel(con
   }
 
   l += shfl_xor(l, 32);
-  if (rw + l31 >= a.R) return;
+  const bool own = rw + l31 < a.R;
   if (a.S > 1) {
+    if (!own) return;
     const long pr = ((long)z * a.BH + bh) * a.R + row;
     if (half == 0) {
       a.mpart[pr] = m;
@@ -330,25 +410,40 @@ __global__ __launch_bounds__(kThreads, D == 256 ? 1 : 2) void prefill_kernel(con
     return;
   }
   const float inv = 1.0f / l;
-  u16* op = a.out + (((long)b * a.Hk * a.gqa + hq) * a.M + pos) * D + 4 * half;
+  float zero = 0.f;  // NaN once an output is not finite
+  if (own) {
+    u16* op = a.out + (((long)b * a.Hk * a.gqa + hq) * a.M + pos) * D + 4 * half;
 #pragma unroll
-  for (int d = 0; d < ND; ++d)
+    for (int d = 0; d < ND; ++d)
 #pragma unroll
-    for (int g = 0; g < 4; ++g)
-      *reinterpret_cast<u32x2_t*>(op + 32 * d + 8 * g) =
-          u32x2_t{attn::pack2<T>(o[d][4 * g] * inv, o[d][4 * g + 1] * inv),
-                  attn::pack2<T>(o[d][4 * g + 2] * inv, o[d][4 * g + 3] * inv)};
+      for (int g = 0; g < 4; ++g) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) zero = __builtin_fmaf(o[d][4 * g + r], 0.f, zero);
+        *reinterpret_cast<u32x2_t*>(op + 32 * d + 8 * g) =
+            u32x2_t{attn::pack2<T>(o[d][4 * g] * inv, o[d][4 * g + 1] * inv),
+                    attn::pack2<T>(o[d][4 * g + 2] * inv, o[d][4 * g + 3] * inv)};
+      }
+  }
+  // a denominator that is not a number came from the scores, and leaves NaN as it should
+  unsigned long long bad = __builtin_amdgcn_ballot_w64(zero != 0.f && l > 0.f && l < __builtin_inff());
+  if (!bad) return;
+  __threadfence_block();  // the outputs above are read back by other lanes
+  for (u32 rows = (u32)bad | (u32)(bad >> 32); rows; rows &= rows - 1) {
+    const int i = __builtin_ctz(rows);
+    auto of = [&](float x) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), i)); };
+    plain_row<T, D>(a, bh, rw + i, of(m), of(l));
+  }
 }
 
 // out = sum_z 2^(m_z - m) o_z / sum_z 2^(m_z - m) l_z over the key splits; 4 outputs a thread.
 // A split that saw none of a row's keys has m = kLowest and l = 0.
-template <class T>
-__global__ __launch_bounds__(256) void combine_kernel(const Args a, int D) {
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  const int per = D / 4;
-  const long row = i / per, rows = (long)a.BH * a.R;
-  if (row >= rows) return;
-  const int d = (int)(i - row * per) * 4;
+template <class T, int D>
+__global__ __launch_bounds__(256) void combine_kernel(const Args a) {
+  constexpr int per = D / 4;  // threads of a row
+  const long i = (long)blockIdx.x * 256 + threadIdx.x, rows = (long)a.BH * a.R;
+  const bool own = i / per < rows;
+  const long row = min(i / per, rows - 1);  // threads past the last row repeat it, and store nothing
+  const int d = (int)(i % per) * 4;
   float m = kLowest;
   for (int z = 0; z < a.S; ++z) m = fmaxf(m, a.mpart[z * rows + row]);
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
@@ -364,8 +459,20 @@ __global__ __launch_bounds__(256) void combine_kernel(const Args a, int D) {
   const int bh = (int)(row / a.R), r = (int)(row - (long)bh * a.R);
   const int pos = r / a.gqa, b = bh / a.Hk, hq = (bh - b * a.Hk) * a.gqa + (r - pos * a.gqa);
   const float inv = 1.0f / l;
-  *reinterpret_cast<u32x2_t*>(a.out + (((long)b * a.Hk * a.gqa + hq) * a.M + pos) * D + d) =
-      u32x2_t{attn::pack2<T>(acc[0] * inv, acc[1] * inv), attn::pack2<T>(acc[2] * inv, acc[3] * inv)};
+  if (own)
+    *reinterpret_cast<u32x2_t*>(a.out + (((long)b * a.Hk * a.gqa + hq) * a.M + pos) * D + d) =
+        u32x2_t{attn::pack2<T>(acc[0] * inv, acc[1] * inv), attn::pack2<T>(acc[2] * inv, acc[3] * inv)};
+  const float zero = acc[0] * 0.f + acc[1] * 0.f + acc[2] * 0.f + acc[3] * 0.f;
+  unsigned long long bad = __builtin_amdgcn_ballot_w64(own && zero != 0.f && l > 0.f && l < __builtin_inff());
+  if (!bad) return;
+  __threadfence_block();
+  while (bad) {
+    const int lead = __builtin_ctzll(bad) / per * per;  // first lane of the row
+    bad &= ~((~0ull >> (64 - per)) << lead);
+    auto of = [&](int x) { return __builtin_amdgcn_readlane(x, lead); };
+    plain_row<T, D>(a, of(bh), of(r), __builtin_bit_cast(float, of(__builtin_bit_cast(int, m))),
+                    __builtin_bit_cast(float, of(__builtin_bit_cast(int, l))));
+  }
 }
 
 }  // namespace prefill

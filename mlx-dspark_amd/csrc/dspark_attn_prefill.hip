@@ -65,7 +65,7 @@ int launch(const Args& a, hipStream_t s) {
   const int st = check_launch("prefill attention");
   if (st || a.S == 1) return st;
   const long threads = (long)a.BH * a.R * (D / 4);
-  hipLaunchKernelGGL((combine_kernel<T>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, a, D);
+  hipLaunchKernelGGL((combine_kernel<T, D>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, a);
   return check_launch("prefill attention combine");
 }
 

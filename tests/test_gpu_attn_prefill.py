@@ -168,3 +168,58 @@ def test_small_probabilities_keep_fp32_precision(dev, dtype, d, L):
             bound = (UNIT[dtype] + (3 * gap + 8 + L / 16) * 2.0 ** -24) * ref.abs() + 2.0 ** -25
             worst = float(((out.double() - ref).abs() / bound).max())
             assert worst <= 1, f"gap {gap} {mask}: {worst} of the bound"
+
+
+@pytest.mark.parametrize("b,hq,hk,m,d", [(1, 8, 2, 2048, 64), (1, 8, 2, 1000, 64), (1, 4, 1, 700, 128),
+                                         (1, 2, 1, 400, 256)])
+def test_key_splits_without_keys(dev, b, hq, hk, m, d):
+    """Few KV heads over as many rows as keys split the keys, and the first row tiles see fewer key
+    tiles than there are splits: a split without any has nothing to add."""
+    from dspark_rocm import _lib, fast
+
+    assert _lib.load().dspark_prefill_attention_workspace(b, hq, hk, m, m, d) > 0
+    q, k, v = _inputs(dev, b, hq, hk, m, m, d, torch.bfloat16)
+    out = fast.scaled_dot_product_attention(q, k, v, scale=d ** -0.5, mask="causal")
+    _check(out, q, k, v, d ** -0.5, True)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,hq,hk,m,L,d", [(1, 4, 2, 70, 150, 64), (2, 6, 2, 43, 64, 128), (1, 2, 1, 40, 90, 256),
+                                           (1, 8, 2, 33, 1500, 64), (1, 8, 2, 33, 1500, 128), (1, 5, 1, 19, 1300, 256)])
+def test_values_that_are_not_finite(dev, dtype, b, hq, hk, m, L, d):
+    """An infinite value makes its column infinite in the rows that see its key, a NaN or both signs
+    make it NaN. Rows masked from it keep theirs or, in its tile, are NaN (zero times infinity, as a
+    product over all keys has it); every other output is what it was, to the bit."""
+    from dspark_rocm import fast
+
+    inf, nan = float("inf"), float("nan")
+    q, k, v = _inputs(dev, b, hq, hk, m, L, d, dtype, qscale=0.5)
+    rep, scale, j = hq // hk, d ** -0.5, L - m + 9        # rows 9.. see key j
+    v2 = v.clone()
+    v2[:, 0, j, 0], v2[:, 0, j, 1], v2[:, -1, j, d - 1] = inf, -inf, nan
+    v2[:, 0, 3, 2], v2[:, 0, 4, 2] = inf, -inf
+    v2[:, 0, 2, 4] = -inf
+    for mask in ("causal", None):
+        clean = fast.scaled_dot_product_attention(q, k, v, scale=scale, mask=mask)
+        got = fast.scaled_dot_product_attention(q, k, v2, scale=scale, mask=mask)
+        first = 9 if mask else 0
+        for heads, row, col, value in ((slice(0, rep), first, 0, inf), (slice(0, rep), first, 1, -inf),
+                                       (slice(0, rep), 0, 2, nan), (slice(0, rep), 0, 4, -inf),
+                                       (slice(hq - rep, hq), first, d - 1, nan)):
+            hit, before = got[:, heads, row:, col], got[:, heads, :row, col]
+            assert bool((hit.isnan() if value != value else hit == value).all()), f"column {col} {mask}"
+            assert bool((before.isnan() | (before == clean[:, heads, :row, col])).all())
+            got[:, heads, :, col] = clean[:, heads, :, col]
+        assert torch.equal(got, clean)
+
+
+@pytest.mark.parametrize("d,L", [(64, 100), (128, 1500)])
+def test_values_at_the_end_of_the_range(dev, d, L):
+    """Values whose unnormalised sum passes the largest fp32 number: the mean of them does not."""
+    from dspark_rocm import fast
+
+    q, k, v = _inputs(dev, 1, 4, 2, 20, L, d, torch.bfloat16)
+    v = (v.float().clamp(-3, 3) * 2.0 ** 125).to(torch.bfloat16)
+    v[..., : d // 2] = v[..., : d // 2].abs()
+    out = fast.scaled_dot_product_attention(q, k, v, scale=0.01, mask="causal")
+    _check(out, q, k, v, 0.01, True)
