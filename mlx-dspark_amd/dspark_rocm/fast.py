@@ -44,7 +44,9 @@ def prefill_kernel(q, k, v, scale, mask, sinks) -> bool:
     recording gradients. Every other call keeps the torch ops."""
     if sinks is not None or not (mask is None or (isinstance(mask, str) and mask == "causal")):
         return False
-    if not isinstance(q, torch.Tensor) or not q.is_cuda or q.dim() != 4 or k.dim() != 4 or k.shape != v.shape:
+    if not all(isinstance(t, torch.Tensor) for t in (q, k, v)) or not ops.eager_inference(q, k, v):
+        return False                        # first: a transform's tensors have no data pointer to ask for
+    if q.dim() != 4 or k.dim() != 4 or k.shape != v.shape:
         return False
     B, Hq, qL, D = q.shape
     Hk, L = k.shape[1], k.shape[2]
@@ -59,7 +61,7 @@ def prefill_kernel(q, k, v, scale, mask, sinks) -> bool:
     for t in (q, k, v):
         if t.stride(3) != 1 or t.data_ptr() % 16 or t.stride(2) > 1 << 22 or any(t.stride(i) % 8 for i in range(3)):
             return False
-    return ops.eager_inference(q, k, v)
+    return True
 
 
 def _stock_sdpa(q, k, v, *, scale, mask=None, sinks=None):

@@ -223,3 +223,19 @@ def test_values_at_the_end_of_the_range(dev, d, L):
     v[..., : d // 2] = v[..., : d // 2].abs()
     out = fast.scaled_dot_product_attention(q, k, v, scale=0.01, mask="causal")
     _check(out, q, k, v, 0.01, True)
+
+
+def test_function_transforms_keep_the_torch_ops(dev):
+    """vmap, grad and jvp over the stock entry point, whose tensors have no data pointer."""
+    from dspark_rocm import fast
+
+    q, k, v = _inputs(dev, 3, 4, 2, 20, 40, 64, torch.bfloat16)
+    f = lambda q, k, v: fast.scaled_dot_product_attention(q, k, v, scale=0.1, mask="causal")  # noqa: E731
+    out = torch.vmap(f)(*(t.unsqueeze(1) for t in (q, k, v)))
+    _check(out.squeeze(1).contiguous(), q, k, v, 0.1, True)
+    qg = q.clone().requires_grad_()
+    want, = torch.autograd.grad(f(qg, k, v).float().sum(), qg)
+    assert torch.equal(torch.func.grad(lambda q: f(q, k, v).float().sum())(q), want)
+    primal, tangent = torch.func.jvp(lambda q: f(q, k, v), (q,), (q,))
+    _check(primal, q, k, v, 0.1, True)
+    assert bool(torch.isfinite(tangent).all()) and float(tangent.float().abs().max()) > 0

@@ -149,3 +149,17 @@ def test_capture_and_replay(dev):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, lin(x))
+
+
+def test_function_transforms_keep_the_torch_product(dev):
+    """A map over several weights, whose tensors have no data pointer, and one over rows."""
+    from dspark_rocm.nn import QuantizedLinear
+
+    mats = [_mats(dev, 96, 128, 8, seed=i) for i in range(2)]
+    lin = QuantizedLinear(*mats[0], bits=8)
+    x = _x(dev, 20, 128)
+    w = torch.stack([m[0] for m in mats])
+    out = torch.vmap(lambda w: torch.func.functional_call(lin, {"weight": w}, (x,)))(w)
+    for i in range(2):
+        _check(out[i], x, w[i], *mats[0][1:], 8)
+    _check(torch.vmap(lin)(x), x, *mats[0], 8)
