@@ -133,18 +133,26 @@ def quantized_matmul_multi(x_list, w_list, s_list, b_list, *, group_size: int = 
     return results
 
 
+def _nothing_intercepts() -> bool:
+    """No tracing, dispatch or function mode, function transform or forward-mode level is active.
+    Some of these are asked of names torch keeps to itself; where one of them is gone, the answer
+    cannot be known, and the calls that ask keep the torch ops."""
+    if torch.jit.is_tracing() or torch.compiler.is_compiling():
+        return False
+    try:
+        return not (torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+                    or torch._C._functorch.peek_interpreter_stack() is not None
+                    or torch.autograd.forward_ad._current_level >= 0)
+    except AttributeError:
+        return False
+
+
 def eager_inference(*ts: torch.Tensor) -> bool:
     """Whether a call on these tensors may go straight to a kernel that autograd, tracing, tensor
     subclasses and function transforms do not see: plain tensors on one ROCm device, nothing that
     records gradients or tangents, no dispatch or function mode and no transform active."""
     first = ts[0]
-    if not first.is_cuda or torch.jit.is_tracing() or torch.compiler.is_compiling():
-        return False
-    if torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack():
-        return False
-    if torch._C._functorch.peek_interpreter_stack() is not None:
-        return False
-    if torch.autograd.forward_ad._current_level >= 0:
+    if not first.is_cuda or not _nothing_intercepts():
         return False
     grad = torch.is_grad_enabled()
     return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.device == first.device
