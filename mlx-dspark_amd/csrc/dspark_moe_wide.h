@@ -57,17 +57,24 @@ __device__ __forceinline__ u32 field_at(const char* w, int n, int k, int K) {
   return BITS == 4 ? (v >> (4 * (k & 1))) & 15u : v;
 }
 
-// One output as the dequantized product in fp32, for outputs whose factored sums are not finite
+// Exact fp32 value of one weight of expert e as an elementwise dequantization rounds it
 template <int BITS, bool PW>
-__device__ float moe_plain_dot(const MoeWideArgs& a, int e, int which, const u16* xr, int n) {
+__device__ __forceinline__ float moe_dequant_at(const MoeWideArgs& a, int e, int which, int n, int k) {
 #pragma clang fp contract(off)
   const char* w = a.w[which] + (long)e * a.N * a.K * BITS / 8;
-  const long sb = ((long)e * a.N + n) * a.G;
-  float acc = 0.f;
-  for (int k = 0; k < a.K && acc == acc; ++k) {
-    const float p = bf2f(a.s[which][sb + (k >> 6)]) * (float)field_at<BITS, PW>(w, n, k, a.K);
-    acc = __builtin_fmaf(bf2f(xr[k]), p + bf2f(a.b[which][sb + (k >> 6)]), acc);
-  }
+  const long g = ((long)e * a.N + n) * a.G + (k >> 6);
+  const float p = bf2f(a.s[which][g]) * (float)field_at<BITS, PW>(w, n, k, a.K);
+  return p + bf2f(a.b[which][g]);
+}
+
+// One output as the dequantized product in fp32, by a lane or (where its row has terms that are not
+// finite) the sum of those; for outputs whose factored sums are not finite
+template <int BITS, bool PW>
+__device__ __forceinline__ float moe_plain(const MoeWideArgs& a, int e, int which, const u16* xr, int n, bool take) {
+  auto weight = [&](int k) { return moe_dequant_at<BITS, PW>(a, e, which, n, k); };
+  float acc;
+  if (!infinite_terms(xr, a.K, take, acc, weight) && take)
+    for (int k = 0; k < a.K && acc == acc; ++k) acc = __builtin_fmaf(bf2f(xr[k]), weight(k), acc);
   return acc;
 }
 
@@ -149,20 +156,21 @@ __global__ __launch_bounds__(kThreads, MT == 2 && BITS == 4 ? 3 : 2) void moe_wi
         if (m < tile.rows && n < a.N) a.y[(long)(tile.p0 + m) * a.ldy + n] = h(v, u);
       }
     }
-  if (bad) {  // the factored sums of an infinite x: outputs that are not finite (a gate or up value
-              // that is not finite leaves one) again from the plain products
+  // the factored sums of an infinite x: outputs that are not finite (a gate or up value that is not
+  // finite leaves one) again from the plain products
+  if (!__builtin_amdgcn_ballot_w64(bad)) return;
+  __threadfence_block();  // the wave's outputs are read back by other lanes
+  const int n = n0 + wave * 16 * NW + lane;
 #pragma unroll 1
-    for (int i = 0; i < 4 * MT * NW; ++i) {
-      const int m = 16 * (i / (4 * NW)) + 4 * q + (i / NW) % 4, n = n0 + wave * 16 * NW + (i % NW) * 16 + c16;
-      if (m >= tile.rows || n >= a.N) continue;
-      u16* y = a.y + (long)(tile.p0 + m) * a.ldy + n;
-      if (!not_finite(bf2f(*y))) continue;
-      const u16* xr = a.x + (long)src(m) * a.ldx;
-      float d[2];
+  for (int m = 0; m < min(16 * MT, tile.rows); ++m) {
+    u16* y = a.y + (long)(tile.p0 + m) * a.ldy + min(n, a.N - 1);
+    const bool take = lane < 16 * NW && n < a.N && not_finite(bf2f(*y));
+    if (!__builtin_amdgcn_ballot_w64(take)) continue;
+    const u16* xr = a.x + (long)src(m) * a.ldx;
+    float d[2];
 #pragma unroll 1
-      for (int j = 0; j < (SWIGLU ? 2 : 1); ++j) d[j] = moe_plain_dot<BITS, PW>(a, tile.e, j, xr, n);
-      *y = h(d[0], d[SWIGLU ? 1 : 0]);
-    }
+    for (int j = 0; j < (SWIGLU ? 2 : 1); ++j) d[j] = moe_plain<BITS, PW>(a, tile.e, j, xr, n, take);
+    if (take) *y = h(d[0], d[SWIGLU ? 1 : 0]);
   }
 }
 

@@ -327,9 +327,43 @@ __device__ __forceinline__ float dequant_at(const Args& a, int n, int k) {
   return p + bf2f(a.b[(long)n * a.G + (k >> 6)]);
 }
 
-// One output as the dequantized product in fp32. The factored sums turn an infinite x into a NaN
-// (inf * 0 for a zero field, inf - inf with the bias term) where the dequantized product is
-// infinite, so outputs that are not finite are computed again this way.
+// The factored sums turn an infinite x into a NaN (inf * 0 for a zero field, inf - inf with the bias
+// term) where the dequantized product is infinite, so outputs that are not finite are computed again.
+// Where the row of x has values that are not finite, their terms are the output: acc becomes the sum of
+// x[k] weight(k) over them, for the lanes of a wave (one output each, all of row xr) that take part.
+// False if the row has none. An infinity in one row of 93 x 17408 x 5120, 4-bit: 65 us, as without; in
+// every row 88; with each output's whole product by its lane 6.9 and 134 ms.
+template <class W>
+__device__ __forceinline__ bool infinite_terms(const u16* xr, int K, bool take, float& acc, W weight) {
+  const int lane = threadIdx.x & 63;
+  acc = 0.f;
+  bool found = false;
+#pragma unroll 1
+  for (int k0 = 0; k0 < K; k0 += 512) {
+    const int k = k0 + 8 * lane;
+    u32 mine = 0;  // bit j: x[k + j] is not finite
+    if (k < K) {
+      const u32x4_t v = ldg128(xr + k);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        mine |= ((v[j >> 1] >> (16 * (j & 1))) & 0x7F80u) == 0x7F80u ? 1u << j : 0u;
+    }
+#pragma unroll 1
+    for (unsigned long long any = __builtin_amdgcn_ballot_w64(mine != 0); any; any &= any - 1) {
+      const int src = __builtin_ctzll(any);
+      found = true;
+#pragma unroll 1
+      for (u32 bits = __builtin_amdgcn_readlane((int)mine, src); bits; bits &= bits - 1) {
+        const int kk = k0 + 8 * src + __builtin_ctz(bits);
+        if (take) acc = __builtin_fmaf(bf2f(xr[kk]), weight(kk), acc);
+        if (!__builtin_amdgcn_ballot_w64(take && acc == acc)) return true;  // all NaN
+      }
+    }
+  }
+  return found;
+}
+
+// One output as the dequantized product in fp32
 template <int BITS>
 __device__ float plain_dot(const Args& a, int m, int n) {
   float acc = 0.f;
@@ -343,6 +377,15 @@ __device__ __forceinline__ bool not_finite(float v) { return !(__builtin_fabsf(v
 __device__ __forceinline__ u16 finish(const Args& a, float v, int n) {
   const u16 r = f2bf(v);
   return a.bias ? f2bf(bf2f(r) + bf2f(a.bias[n])) : r;  // the module's bias is added to the bf16 product
+}
+
+// Outputs y[m, n] again, by one wave: m is the wave's, n the lane's, take whether it has one.
+template <int BITS>
+__device__ __forceinline__ void plain_outputs(const Args& a, int m, int n, bool take) {
+  float acc;
+  if (!infinite_terms(a.x + (long)m * a.ldx, a.K, take, acc, [&](int k) { return dequant_at<BITS>(a, n, k); }) && take)
+    acc = plain_dot<BITS>(a, m, n);
+  if (take) a.y[(long)m * a.ldy + n] = finish(a, acc, n);
 }
 
 template <int BITS, int MT, int NT>
@@ -417,13 +460,13 @@ __global__ __launch_bounds__(kThreads, 2) void wide_kernel(const Args a) {
         if (m < a.M && n < a.N) a.y[(long)m * a.ldy + n] = finish(a, acc[mt][nt][r], n);
       }
     }
-  if (bad) {  // this lane's outputs again, those that are not finite from the plain product
+  if (!__builtin_amdgcn_ballot_w64(bad)) return;
+  __threadfence_block();  // the wave's outputs are read back by other lanes
+  const int n = n0 + wave * 16 * NT + lane;
 #pragma unroll 1
-    for (int i = 0; i < 4 * MT * NT; ++i) {
-      const int m = m0 + 16 * (i / (4 * NT)) + 4 * q + (i / NT) % 4, n = n0 + wave * 16 * NT + (i % NT) * 16 + c16;
-      if (m >= a.M || n >= a.N || !not_finite(bf2f(a.y[(long)m * a.ldy + n]))) continue;
-      a.y[(long)m * a.ldy + n] = finish(a, plain_dot<BITS>(a, m, n), n);
-    }
+  for (int m = m0; m < min(m0 + 16 * MT, a.M); ++m) {
+    const bool take = lane < 16 * NT && n < a.N && not_finite(bf2f(a.y[(long)m * a.ldy + min(n, a.N - 1)]));
+    if (__builtin_amdgcn_ballot_w64(take)) plain_outputs<BITS>(a, m, n, take);
   }
 }
 
@@ -431,25 +474,38 @@ __global__ __launch_bounds__(kThreads, 2) void wide_kernel(const Args a) {
 template <int BITS>
 __global__ __launch_bounds__(256) void wide_reduce_kernel(const Args a) {
   const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4, total = (long)a.M * a.N;
-  if (i >= total) return;
   float v[4] = {0.f, 0.f, 0.f, 0.f};
-  const int cnt = (int)min(4L, total - i);
+  const int cnt = (int)max(0L, min(4L, total - i));
   if (a.N % 4 == 0) {
-    for (int z = 0; z < a.S; ++z) {
-      const f32x4_t p = *reinterpret_cast<const f32x4_t*>(a.part + z * total + i);
+    if (cnt)
+      for (int z = 0; z < a.S; ++z) {
+        const f32x4_t p = *reinterpret_cast<const f32x4_t*>(a.part + z * total + i);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] += p[j];
-    }
+        for (int j = 0; j < 4; ++j) v[j] += p[j];
+      }
   } else {
     for (int z = 0; z < a.S; ++z)
       for (int j = 0; j < cnt; ++j) v[j] += a.part[z * total + i + j];
   }
+  u32 bad = 0;  // bit j: output i + j is not finite
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     if (j >= cnt) break;
     const int m = (int)((i + j) / a.N), n = (int)((i + j) - (long)m * a.N);
-    const float f = not_finite(v[j]) ? plain_dot<BITS>(a, m, n) : v[j];
-    a.y[(long)m * a.ldy + n] = finish(a, f, n);
+    a.y[(long)m * a.ldy + n] = finish(a, v[j], n);
+    bad |= not_finite(v[j]) ? 1u << j : 0u;
+  }
+  if (!__builtin_amdgcn_ballot_w64(bad != 0)) return;
+#pragma unroll 1
+  for (int j = 0; j < 4; ++j) {
+    const int m = (int)((i + j) / a.N), n = (int)((i + j) - (long)m * a.N);
+    // the lanes of one row of x at a time
+    for (unsigned long long left = __builtin_amdgcn_ballot_w64((bad >> j) & 1); left;) {
+      const int row = __builtin_amdgcn_readlane(m, __builtin_ctzll(left));
+      const bool take = ((bad >> j) & 1) && m == row;
+      left &= ~__builtin_amdgcn_ballot_w64(take);
+      plain_outputs<BITS>(a, row, n, take);
+    }
   }
 }
 

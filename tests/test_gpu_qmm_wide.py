@@ -163,3 +163,56 @@ def test_function_transforms_keep_the_torch_product(dev):
     for i in range(2):
         _check(out[i], x, w[i], *mats[0][1:], 8)
     _check(torch.vmap(lin)(x), x, *mats[0], 8)
+
+
+def _us(f):
+    f()
+    best = float("inf")
+    for _ in range(3):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        f()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b) * 1e3)
+    return best
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("m,n,k", [(70, 300, 1088), (96, 5120, 2048), (300, 8192, 1024)])   # also one slice, K slices
+def test_infinite_rows_cost_no_more_than_their_terms(dev, m, n, k, bits):
+    """An infinity in every row: each output is its term (a NaN where the weight is zero), and the call
+    stays within 20 times one without (about 1.3 measured; a whole product per output took 1000)."""
+    from dspark_rocm import ops, quant
+
+    w, s, b = _mats(dev, n, k, bits)
+    s[5], b[5] = 0, 0
+    x = _x(dev, m, k)
+    at = torch.arange(m, device=dev) * 7 % k
+    x2 = x.clone()
+    x2[torch.arange(m, device=dev), at] = float("inf")
+    call = lambda x: ops.quantized_matmul_wide(x, w, s, b, bits=bits)  # noqa: E731
+    got, deq = call(x2).float(), quant.dequantize(w, s, b, 64, bits)
+    want = float("inf") * deq[:, at].t()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0))
+    assert _us(lambda: call(x2)) <= 20 * _us(lambda: call(x)) + 100
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("m,n,k", [(40, 200, 192), (96, 640, 2048)])
+def test_factored_sums_that_overflow_are_the_plain_product(dev, m, n, k, bits):
+    """Inputs near the end of the range, whose products with whole fields overflow."""
+    from dspark_rocm import ops
+
+    w, s, b = _mats(dev, n, k, bits)
+    x = _x(dev, m, k)
+    x[3, 5], x[9, 17], x[9, 18] = 2.0 ** 125, 2.0 ** 124, -(2.0 ** 124)
+    ref, _ = _reference(x, w, s, b, bits)
+    assert float(ref.abs().max()) < 2.0 ** 127
+    got = ops.quantized_matmul_wide(x, w, s, b, bits=bits)
+    big = [3, 9]
+    deq = (x[big].double().abs() @ (_reference(torch.eye(k, device=dev), w, s, b, bits)[0]).abs())
+    assert bool(((got[big].double() - ref[big]).abs() <= 2.0 ** -8 * ref[big].abs() + k * 2.0 ** -23 * deq).all())
+    keep = torch.ones(m, dtype=torch.bool, device=dev)
+    keep[big] = False
+    _check(got[keep], x[keep], w, s, b, bits)
