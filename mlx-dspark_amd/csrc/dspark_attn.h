@@ -34,6 +34,8 @@
 //     bf16/fp16 cache of the dequantized values.
 #pragma once
 
+#include <algorithm>
+
 #include "dspark_qmm_core.h"
 
 namespace dspark {
@@ -115,7 +117,7 @@ struct Plan {
   int R, RT, RP, WV, KS, PF, NRG, chunk, NB;
 };
 
-inline Plan make_plan(long B, long Hq, long Hk, long Mq, long D, long L) {
+inline Plan make_plan(long B, long Hq, long Hk, long Mq, long D, long L, bool quantized) {
   Plan p{};
   p.R = (int)((Hq / Hk) * Mq);
   p.RT = (p.R + 15) / 16;
@@ -137,19 +139,32 @@ inline Plan make_plan(long B, long Hq, long Hk, long Mq, long D, long L) {
   const long heads = B * Hk * p.NRG;
   const long target = (p.WV == 8 || D == 256) ? 256 : 512;
   long nb = (target + heads - 1) / heads;
-  // Head dim 256 keeps 128 keys (four of its tiles) beyond that, where few KV heads otherwise leave
-  // half the CUs idle: 24/4 heads, 6 rows, 10007 keys 29.9 -> 26.9 us over an 8-bit cache, 20.3 ->
-  // 18.7 over bf16; 16 rows 53.7 -> 45.6 and 27.0 -> 25.0; but over 5000 keys 16 rows (more than 4
-  // row tiles) lose more to the partials than they gain (8-bit 31.4 -> 36.6).
-  const bool short_blocks = L < 4096 || (D == 256 && (p.RT <= 4 || L >= 8192));
-  const long min_keys = L <= 1280 ? 64 : (short_blocks ? 128 : 256);
-  const long max_nb = (L + min_keys - 1) / min_keys;
-  if (nb > max_nb) nb = max_nb;
+  const long min_keys = L <= 1280 ? 64 : (L < 4096 ? 128 : 256);
+  nb = std::min(nb, (L + min_keys - 1) / min_keys);
+  // Head dim 256 goes on with 128 keys (four of its tiles) beyond that, as few KV heads leave CUs idle
+  // (24/4 heads over an 8-bit cache: 8 rows, 6000 keys 28.1 -> 22.6 us; 16 rows, 10007 keys 53 -> 45).
+  // But no CU gets a second workgroup by it (18/3, one row, 16500 8-bit keys: 27.9 in 65 blocks, 38.7
+  // in 86), nor the combine over a bf16 cache more than 192 blocks (4/1, 8 rows, 32768 keys: 21.6 in
+  // 128, 23.2 in 256). More than 4 row tiles (6 waves) lose more to the partials below 8192 keys (24/4,
+  // 16 rows, 5000 8-bit keys: 31.4 and 36.6), and over quantized caches past 128 workgroups where blocks
+  // of 256 keys are no more than that (12/2, 16 rows, 9000 keys: 30.7 and 35.7).
+  if (D == 256 && L >= 4096) {
+    long short_nb = std::min(256 / heads, (L + 127) / 128);
+    if (!quantized) short_nb = std::min(short_nb, 192L);
+    const bool six_waves = p.RT > 4;
+    const bool crowded = quantized && p.NRG == 1 && heads * ((L + 127) / 128) > 128 && heads * (L / 256) <= 128;
+    if (!six_waves || (L >= 8192 && !crowded)) nb = std::max(nb, short_nb);
+  }
   // Somewhat more than one workgroup a CU leaves most CUs waiting for those with two: one each
-  // instead (32/8 heads x 128, 16 rows: 8500 keys 19.3 -> 16.8 us, 10007 keys 20.3 -> 17.6, over an
-  // 8-bit cache 27.2 -> 23.1). Not beyond one and a half (14000 keys, 6 rows, 8-bit: 22.0 -> 22.9),
-  // nor for the single row tile of a plain decode step (12000 keys: 17.1 -> 19.1).
-  if (D <= 128 && target == 512 && p.RT > 1 && heads * nb > 256 && heads * nb <= 384) nb = (256 + heads - 1) / heads;
+  // instead (32/8 heads x 128, 16 rows, 10007 keys: bf16 20.3 -> 17.7 us, over an 8-bit cache 26.3 ->
+  // 22.2), if those beyond 256 are whole blocks (8200 8-bit keys, 5 rows: 16.4 in 33 blocks, 17.6 in 26).
+  // Not beyond one and a half, nor for the single row tile of a plain decode step (12000 keys: 17.1 -> 19.1).
+  if (D <= 128 && target == 512 && p.RT > 1 && heads * (L / min_keys) > 256 && heads * nb <= 384) {
+    const long n = (256 + heads - 1) / heads, c = ((L + n - 1) / n + 63) / 64 * 64;
+    // where 256 is no multiple of the heads, what is over 256 has to be short blocks too (48/12, 8 rows,
+    // 7000 keys: 16.9 in 28 blocks, 18.4 in 22; 28/7, 10007 8-bit keys 21.4 in 40, 18.9 in 32)
+    if (heads * (L / c) <= 256 && (heads * ((L + c - 1) / c) <= 256 || 2 * (L % c) <= c)) nb = n;
+  }
   if (nb < 1) nb = 1;
   if (p.WV == 4 && D <= 128 && heads * nb < 256) p.KS = 2;
   long chunk = (L + nb - 1) / nb;

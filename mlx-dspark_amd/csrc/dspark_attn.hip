@@ -42,7 +42,7 @@ struct Common {
   size_t workspace_bytes;
 };
 
-int prepare(const Common& c, AttnArgs& a, Plan& p) {
+int prepare(const Common& c, bool quantized, AttnArgs& a, Plan& p) {
   if (!c.q || !c.out || !c.out_strides) return fail(DSPARK_ERR_ARG, "verify_attention: null pointer");
   int st = check_shape(c.B, c.Hq, c.Mq, c.D, c.Hk, c.L);
   if (st) return st;
@@ -51,7 +51,7 @@ int prepare(const Common& c, AttnArgs& a, Plan& p) {
   if (!aligned(c.q, 16) || !aligned(c.out, 8))
     return fail(DSPARK_ERR_ALIGN, "verify_attention: q must be 16-byte aligned, out 8-byte aligned");
   const long DI = instance_d(c.D);
-  p = make_plan(c.B, c.Hq, c.Hk, c.Mq, DI, c.L);
+  p = make_plan(c.B, c.Hq, c.Hk, c.Mq, DI, c.L, quantized);
   const size_t need = partial_bytes(p, c.B, c.Hk, DI);
   if (need && (!c.workspace || c.workspace_bytes < need))
     return fail(DSPARK_ERR_WORKSPACE, "verify_attention: workspace %zu < %zu bytes", c.workspace_bytes, need);
@@ -111,7 +111,7 @@ int plain_impl(int dtype, const Common& c, const void* k, const void* v, const i
   if (!k || !v || !k_strides || !v_strides) return fail(DSPARK_ERR_ARG, "verify_attention: null pointer");
   AttnArgs a{};
   Plan p{};
-  if ((st = prepare(c, a, p))) return st;
+  if ((st = prepare(c, false, a, p))) return st;
   if (!aligned(k, 16) || !aligned(v, 16)) return fail(DSPARK_ERR_ALIGN, "verify_attention: k/v must be 16-byte aligned");
   if ((st = check_strides(k_strides, 8, "K")) || (st = check_strides(v_strides, 8, "V"))) return st;
   // the kernels address a key tile with 32-bit byte offsets from its first key
@@ -140,7 +140,9 @@ extern "C" size_t dspark_verify_attention_workspace(int64_t B, int64_t Hq, int64
                                                     int64_t L_total) {
   if (check_shape(B, Hq, Mq, D, Hk, L_total)) return 0;
   const long DI = instance_d(D);
-  return partial_bytes(make_plan(B, Hq, Hk, Mq, DI, L_total), B, Hk, DI);
+  // plain and quantized caches may differ in their blocks
+  return std::max(partial_bytes(make_plan(B, Hq, Hk, Mq, DI, L_total, false), B, Hk, DI),
+                  partial_bytes(make_plan(B, Hq, Hk, Mq, DI, L_total, true), B, Hk, DI));
 }
 
 extern "C" int dspark_verify_attention_plan(int64_t B, int64_t Hq, int64_t Hk, int64_t Mq, int64_t D,
@@ -148,7 +150,7 @@ extern "C" int dspark_verify_attention_plan(int64_t B, int64_t Hq, int64_t Hk, i
   if (!out) return fail(DSPARK_ERR_ARG, "verify_attention_plan: null output");
   const int st = check_shape(B, Hq, Mq, D, Hk, L_total);
   if (st) return st;
-  const Plan p = make_plan(B, Hq, Hk, Mq, instance_d(D), L_total);
+  const Plan p = make_plan(B, Hq, Hk, Mq, instance_d(D), L_total, false);
   out[0] = p.R;
   out[1] = p.RP;
   out[2] = p.NRG;
@@ -161,7 +163,7 @@ extern "C" int dspark_verify_attention_plan(int64_t B, int64_t Hq, int64_t Hk, i
 extern "C" int64_t dspark_verify_attention_blocks(int64_t B, int64_t Hq, int64_t Hk, int64_t Mq, int64_t D,
                                                   int64_t L_total) {
   if (check_shape(B, Hq, Mq, D, Hk, L_total)) return -1;
-  return make_plan(B, Hq, Hk, Mq, instance_d(D), L_total).NB;
+  return make_plan(B, Hq, Hk, Mq, instance_d(D), L_total, false).NB;
 }
 
 extern "C" int dspark_verify_attention_typed(int dtype, const void* q, int64_t B, int64_t Hq, int64_t Mq, int64_t D,
@@ -214,7 +216,7 @@ extern "C" int dspark_verify_attention_quantized(
   const Common c{q, B, Hq, Mq, D, Hk, L_total, scale, causal, nullptr, out, out_strides, workspace, workspace_bytes};
   AttnArgs a{};
   Plan p{};
-  if ((st = prepare(c, a, p))) return st;
+  if ((st = prepare(c, true, a, p))) return st;
   // word rows are read as 16-byte chunks (K) and 8- or 4-byte pieces (V); scales and biases
   // as single values
   if (!aligned(k_words, 16) || !aligned(v_words, 16) || !aligned(k_scales, 2) || !aligned(k_biases, 2) ||
