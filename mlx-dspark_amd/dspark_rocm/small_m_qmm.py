@@ -9,9 +9,11 @@ The reference's entry points (small_m_qmm.py:57-243) on torch modules:
   (small_m_qmm.py:71-80). Exit restores that method, so the scope nests with others holding
   the class (tests/test_small_m_qmm.py:159-171).
 * ``measure_shapes(*models)`` is the load-time gate (small_m_qmm.py:142-230): per distinct
-  shape, the kernel must agree with the stock path (``max|d| <= 0.02 * max(max|stock|, 1)``
-  at M in {lo, 8, 12, hi}) and win a race over the model's own same-shape layers: 1.15x at
-  M = 8 and 12, and no worse than 0.97x at the bottom of the window when it starts below 6.
+  shape, the kernel must agree with the dequantized fp32 product (``max|d| <= 0.02 * max(max|ref|, 1)``
+  at M in {lo, 8, 12, hi}) and win a race against it over the model's own same-shape layers: 1.15x at
+  M = 8 and 12, and no worse than 0.97x at the bottom of the window when it starts below 6. At the
+  same widths it must be no worse than 0.97x against the stock path itself, where that is not this
+  product but the matrix-core kernel for many rows.
   The race is :func:`dspark_rocm.gate.speedup` (HIP events). A shape whose kernel raises is
   off; nothing here raises.
 """
@@ -105,8 +107,8 @@ def _probe_x(K: int, M: int, gen: torch.Generator, device) -> torch.Tensor:
 
 
 def numerics_ok(mod, seed: int = 0) -> bool:
-    """Kernel vs stock at M in {lo, 8, 12, hi}: ``max|kernel - stock| <= 0.02 * max(max|stock|, 1)``
-    (the module's own bias, if any, is left out of both)."""
+    """Kernel vs dequantized product at M in {lo, 8, 12, hi}: ``max|kernel - ref| <= 0.02 *
+    max(max|ref|, 1)`` (the module's own bias, if any, is left out of both)."""
     K = _in_features(mod)
     lo, hi = _sk.WINDOW[int(mod.bits)]
     gen = torch.Generator(device=mod.weight.device)
@@ -114,11 +116,11 @@ def numerics_ok(mod, seed: int = 0) -> bool:
     bias = getattr(mod, "bias", None)
     for M in sorted({lo, 8, 12, hi}):
         x = _probe_x(K, M, gen, mod.weight.device)
-        stock = _orig_call(mod, x).float()
+        ref = mod.torch_product(x).float()
         if bias is not None:
-            stock = stock - bias.float()
-        scale = max(float(stock.abs().max()), 1.0)
-        if not gate.max_abs_diff(_kernel_rows(mod, x), stock) <= _REL_TOL * scale:
+            ref = ref - bias.float()
+        scale = max(float(ref.abs().max()), 1.0)
+        if not gate.max_abs_diff(_kernel_rows(mod, x), ref) <= _REL_TOL * scale:
             return False
     return True
 
@@ -131,14 +133,24 @@ def _bars(bits: int) -> list[gate.Bar]:
     return bars
 
 
-def _race(mods: list, rows: int, gen: torch.Generator) -> float:
-    """Dequantized product / kernel time at ``rows`` rows over chains rotating through ``mods``: the
-    bars were set for it (the stock path's own matrix-core product is built for prefill widths and
-    behind these kernels in all of their window)."""
+def _chains(mods: list, rows: int, gen: torch.Generator, other):
     x = _probe_x(_in_features(mods[0]), rows, gen, mods[0].weight.device)
     seq = [mods[t % len(mods)] for t in range(_CHAIN)]
-    return gate.speedup([lambda m=m: m.torch_product(x) for m in seq],
+    return gate.speedup([lambda m=m: other(m, x) for m in seq],
                         [lambda m=m: _kernel_rows(m, x) for m in seq], repeat=_EVALS - 1)
+
+
+def _race(mods: list, rows: int, gen: torch.Generator) -> float:
+    """Dequantized product / kernel time at ``rows`` rows over chains rotating through ``mods``: what the
+    bars were set for."""
+    return _chains(mods, rows, gen, lambda m, x: m.torch_product(x))
+
+
+def _stock_race(mods: list, rows: int, gen: torch.Generator) -> float:
+    """The same for what the modules run outside the scope. Over 21 shapes from [100, 64] to
+    [151936, 4096] and rows 1 to 16 it is 1.7 to 2.2 up to 50M weights, where calls cost more on the
+    host than on the GPU, and 1.0 to 1.4 (8 bits) or 1.3 to 1.8 (4 bits) above."""
+    return _chains(mods, rows, gen, _orig_call)
 
 
 def _shape_verdict(key: str, mods: list, verbose: bool) -> bool:
@@ -150,10 +162,12 @@ def _shape_verdict(key: str, mods: list, verbose: bool) -> bool:
     gen.manual_seed(0)
     results = [(bar, _race(mods, bar.rows, gen)) for bar in _bars(int(mods[0].bits))]
     on = all(bar.met(r) for bar, r in results)
+    behind = [f"M={bar.rows} {r:.2f}x stock" for bar, r in ((bar, _stock_race(mods, bar.rows, gen)) for bar, _ in results)
+              if r < _EDGE_MIN] if on else []
     if verbose:
-        detail = ", ".join(f"M={bar.rows} {r:.2f}x (>= {bar.min_speedup})" for bar, r in results)
-        print(f"  small-M qmm: {key} {detail}: {'on' if on else 'off'}", flush=True)
-    return on
+        detail = ", ".join([f"M={bar.rows} {r:.2f}x (>= {bar.min_speedup})" for bar, r in results] + behind)
+        print(f"  small-M qmm: {key} {detail}: {'on' if on and not behind else 'off'}", flush=True)
+    return on and not behind
 
 
 def _by_shape(models) -> dict[str, list]:
@@ -166,7 +180,7 @@ def _by_shape(models) -> dict[str, list]:
 
 
 def measure_shapes(*models, verbose: bool = False) -> list[str]:
-    """Shape keys whose kernel path agrees with the stock path and wins the race here."""
+    """Shape keys whose kernel agrees with the dequantized product and wins the races here."""
     won = []
     for key, mods in _by_shape(models).items():
         try:

@@ -243,3 +243,21 @@ def test_apply_wiring_measures_and_routes(dev, tmp_path, monkeypatch):
         assert small_m_qmm.active() and multirow_attn.active()
         mod = model(ids_t.to(dev), cb)
     assert_rms_close(_np(mod[0]), _np(fused[0]), 5e-2, "module path under the applied scopes vs fused")
+
+
+def test_small_m_gate_sees_the_path_it_replaces(dev, monkeypatch):
+    """Outside the scope a bf16 call runs the matrix-core kernel for many rows: a small-M kernel slower
+    than that is refused though it beats the dequantized product, and a drift the two share is seen."""
+    from dspark_rocm import ops
+    from dspark_rocm import small_m_qmm as sm
+
+    mods = torch.nn.ModuleList([_ql(dev, 8, 4096, 4096, 40 + i) for i in range(4)])
+    real = sm._kernel_rows
+    assert sm.measure_shapes(mods) == [sm.shape_key(mods[0])]
+    monkeypatch.setattr(sm, "_kernel_rows", lambda mod, x: [real(mod, x) for _ in range(5)][0])
+    gen = torch.Generator(device=dev)
+    assert sm._race(list(mods), 8, gen) > sm._MIN_GAIN and sm.measure_shapes(mods) == []
+    drift = lambda f: lambda *a, **k: f(*a, **k) * 1.05 + 0.5  # noqa: E731
+    monkeypatch.setattr(ops, "quantized_matmul_wide", drift(ops.quantized_matmul_wide))
+    monkeypatch.setattr(sm, "_kernel_rows", drift(real))
+    assert not sm.numerics_ok(mods[0])
