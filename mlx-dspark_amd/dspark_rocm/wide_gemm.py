@@ -157,21 +157,34 @@ def _probe_x(mod, M: int, gen: torch.Generator) -> torch.Tensor:
     return torch.randn((M, _in_features(mod)), generator=gen, device=mod.weight.device).to(mod.scales.dtype)
 
 
+def _one_row(mod) -> torch.Tensor:
+    return torch.zeros((1, _in_features(mod)), dtype=mod.scales.dtype, device=mod.weight.device)
+
+
+def _stock_is_kernel(mod, x: torch.Tensor, exact: bool) -> bool:
+    """Whether the stock path and the exact wide path are one kernel for this call."""
+    return exact and mod.wide_kernel(x)
+
+
 def _agrees(mod, M: int, exact: bool = True, seed: int = 0, draws: int = 2) -> bool:
     """Whether the wide path gives the stock path's result for this weight at ``M`` rows on
     ``draws`` random inputs: bit for bit, or (``exact=False``) within the qmm bar. One lucky
-    match proves little, hence two draws by default (wide_gemm.py:262-280)."""
+    match proves little, hence two draws by default (wide_gemm.py:262-280). Where both are the
+    matrix-core kernel, it also has to be within the qmm bar of the dequantized product."""
     gen = torch.Generator(device=mod.weight.device)
     gen.manual_seed(seed + M)
+
+    def within_bar(ref: torch.Tensor, y: torch.Tensor) -> bool:
+        return gate.max_abs_diff(ref, y) <= REL_TOL * max(float(ref.float().abs().max()), 1.0)
 
     def one_draw() -> bool:
         x = _probe_x(mod, M, gen)
         stock, wide = _orig_call(mod, x), wide_rows(mod, x, exact=exact)
         if stock.shape != wide.shape or not bool(torch.isfinite(wide.float()).all()):
             return False
-        if exact:
-            return torch.equal(stock, wide)
-        return gate.max_abs_diff(stock, wide) <= REL_TOL * max(float(stock.float().abs().max()), 1.0)
+        if _stock_is_kernel(mod, x, exact) and not within_bar(mod.torch_product(x), wide):
+            return False
+        return torch.equal(stock, wide) if exact else within_bar(stock, wide)
 
     return all(one_draw() for _ in range(draws))
 
@@ -211,8 +224,10 @@ def measure_crossover(*models, widths: tuple[int, ...] = (256, 512, 1024, 2048),
 
     The widest weight is raced at every width (widths under :data:`SAFE_MIN_ROWS` never take the
     path); ``min_rows`` is where the run of winning widths that reaches the widest one starts,
-    and the shapes are those that verify there and at every wider width."""
-    lin = widest_quantized_linear(*models)
+    and the shapes are those that verify there and at every wider width. Weights whose stock path
+    is already the wide path's kernel are not raced: there is nothing to win."""
+    lin = max((mod for mod in quantized_linears(*models) if not _stock_is_kernel(mod, _one_row(mod), exact)),
+              key=lambda mod: mod.weight.numel(), default=None)
     if lin is None:
         return None
     gen = torch.Generator(device=lin.weight.device)

@@ -168,3 +168,23 @@ def test_prefill_fills_caches_identically_with_the_wide_path(dev, monkeypatch):
         ka, va = a.fetch()
         kb, vb = b.fetch()
         assert torch.equal(ka, kb) and torch.equal(va, vb)
+
+
+def test_verification_is_against_the_dequantized_product(dev, monkeypatch):
+    """bf16 calls run one kernel with and without the wide path: agreeing with itself verifies
+    nothing, and there is nothing to race."""
+    from dspark_rocm import ops
+    from dspark_rocm import wide_gemm as wg
+
+    lin = _lin_at(dev, torch.bfloat16, 8, n=512, k=1024)
+    half = _lin_at(dev, torch.float16, 8, n=256, k=512)
+    assert wg._agrees(lin, 256) and wg._agrees(half, 256)
+    raced = []
+    monkeypatch.setattr(wg, "_wide_wins", lambda mod, *a: raced.append(mod) or True)
+    assert wg.measure_crossover(torch.nn.Sequential(lin)) is None and raced == []
+    min_rows, keys = wg.measure_crossover(torch.nn.Sequential(lin, half))
+    assert min_rows == 256 and keys == [wg.shape_key(lin), wg.shape_key(half)]
+    assert all(mod is half for mod in raced) and raced
+    real = ops.quantized_matmul_wide
+    monkeypatch.setattr(ops, "quantized_matmul_wide", lambda *a, **k: real(*a, **k) * 1.05 + 0.5)
+    assert wg.verified_shapes([torch.nn.Sequential(lin, half)], 256, widths=()) == [wg.shape_key(half)]
