@@ -149,7 +149,8 @@ int dspark_qmm_dequantize(const uint32_t* w, const void* scales, const void* bia
 
 /*
  * The same product for many rows (prefill widths): y = x . dequant(w)^T for reference-layout w
- * and bf16 scales / biases, any M >= 1, N >= 1, K % 64 == 0. fp32 accumulation over exact
+ * and bf16 scales / biases, any M >= 1, N >= 1, K % 64 == 0, with at most 2^28 group sums (M rows of
+ * K / 64, up to a multiple of 32). fp32 accumulation over exact
  * products, weights never rounded; outputs that are not finite are recomputed as the plain fp32
  * dequantized product. `bias` (nullable, bf16 [N]) is added to the bf16 product, rounded again.
  * x 16-byte aligned with ldx % 8 == 0, w 16-byte aligned. Workspace 256-byte aligned, any

@@ -41,6 +41,9 @@ struct Plan {
   size_t xs_bytes, part_bytes, total;
 };
 
+// Group sums of a row, padded to whole MFMA steps
+inline long padded_groups(long K) { return (K / 64 + 31) / 32 * 32; }
+
 inline size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 
 Plan make_plan(long M, long K, long N, int bits) {
@@ -75,7 +78,7 @@ Plan make_plan(long M, long K, long N, int bits) {
       }
     }
   }
-  p.GP = (int)((G + 31) / 32 * 32);
+  p.GP = (int)padded_groups(K);
   p.xs_bytes = round256((size_t)kPieces * M * p.GP * 2);
   p.part_bytes = p.S > 1 ? round256((size_t)p.S * M * N * 4) : 0;
   p.total = p.xs_bytes + p.part_bytes;
@@ -87,6 +90,9 @@ int check(long M, long K, long N, int bits, int group_size) {
   if (group_size != 64) return fail(DSPARK_ERR_UNSUPPORTED, "qmm_wide: group_size=%d (64)", group_size);
   if (M < 1 || N < 1 || K < 64 || K % 64 || M > (1L << 24) || N > (1L << 24) || K > (1L << 22))
     return fail(DSPARK_ERR_SHAPE, "qmm_wide: M=%ld K=%ld N=%ld", M, K, N);
+  // the group sums take 8 threads each, and a launch has fewer than 2^32
+  if (M * padded_groups(K) > (1L << 28))
+    return fail(DSPARK_ERR_SHAPE, "qmm_wide: M=%ld x %ld group sums (at most 2^28)", M, padded_groups(K));
   return DSPARK_OK;
 }
 
@@ -156,7 +162,7 @@ extern "C" int dspark_qmm_wide(const void* x, int64_t ldx, int64_t M, int64_t K,
   a.ntiles = p.ntiles;
   a.vec = wide::chunk_rows(a.G, scales, biases);
   const long tiles = (long)p.mtiles * p.ntiles * p.S;
-  if (tiles > (1L << 30)) return fail(DSPARK_ERR_SHAPE, "qmm_wide: too many tiles");
+  if (tiles > (1L << 23)) return fail(DSPARK_ERR_SHAPE, "qmm_wide: too many tiles");
   a.per_xcd = (int)((tiles + 7) / 8);
 
   if ((st = wide::launch_group_sums(a.x, ldx, M, a.G, p.GP, xs, s))) return st;

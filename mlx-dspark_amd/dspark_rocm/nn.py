@@ -85,8 +85,9 @@ class QuantizedLinear(nn.Module):
         params = (w, s, b) if bias is None else (w, s, b, bias)
         if not ops.eager_inference(x, *params):     # first: a transform's tensors have no data pointer to ask for
             return False
-        return (x.shape[-1] == k and 0 < x.numel() <= k << 24 and 0 < k <= 1 << 22 and 0 < n <= 1 << 24
-                and k % GROUP == 0 and tuple(s.shape) == (n, k // GROUP) and b.shape == s.shape
+        return (x.shape[-1] == k and 0 < k <= 1 << 22 and 0 < n <= 1 << 24 and k % GROUP == 0 and x.numel() > 0
+                and x.numel() // k * (-(-k // 2048) * 32) <= 1 << 28        # the kernel's group sums
+                and tuple(s.shape) == (n, k // GROUP) and b.shape == s.shape
                 and all(p.dtype == torch.bfloat16 for p in params[1:])
                 and (bias is None or tuple(bias.shape) == (n,))
                 and w.is_contiguous() and w.data_ptr() % 16 == 0)

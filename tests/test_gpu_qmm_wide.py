@@ -216,3 +216,11 @@ def test_factored_sums_that_overflow_are_the_plain_product(dev, m, n, k, bits):
     keep = torch.ones(m, dtype=torch.bool, device=dev)
     keep[big] = False
     _check(got[keep], x[keep], w, s, b, bits)
+
+
+def test_rows_beyond_one_launch_keep_the_torch_product(dev):
+    from dspark_rocm.nn import QuantizedLinear
+
+    lin = QuantizedLinear(*_mats(dev, 8, 64, 8), bits=8)
+    x = _x(dev, 1, 64)
+    assert lin.wide_kernel(x.expand(1 << 23, 64)) and not lin.wide_kernel(x.expand((1 << 23) + 1, 64))
