@@ -310,6 +310,7 @@ class VerifyEngine:
         # The engine's own workspaces, sized once for every launch of a step at up to max_rows
         # rows and any cache length, so a captured step never sees them move.
         self._widths = (hq * d, hk * d, hk * d, H, I, H)     # outputs of q, k, v, o, gate / up, down
+        self._device = self.h.device
         self.qmm_ws = ops.new_qmm_workspace(dev, self._qmm_workspace_need())
         self.accept_ws = torch.zeros(max(ops.argmax_accept_workspace_bytes(max_rows, a.vocab_size), 256),
                                      dtype=torch.uint8, device=dev)
@@ -322,23 +323,19 @@ class VerifyEngine:
 
     def _norm_fits(self, w: torch.Tensor, n: int) -> bool:
         """Whether ``w`` is a norm weight the native step may pass as a bare pointer."""
-        return w.device == self.h.device and w.dtype == torch.bfloat16 and w.shape == (n,) and w.is_contiguous()
+        return w.dtype is torch.bfloat16 and w.numel() == n and w.device == self._device and w.is_contiguous()
 
-    def _cache_fits(self, c, bits: int, need: int) -> bool:
-        """Whether every tensor of cache ``c`` holds ``need`` rows of the model's KV heads, batch 1, on
-        the engine's device, in the type and width its kernels read: the native step passes pointers
-        and strides, and the model's sizes for the rest."""
-        a, bf = self.args, torch.bfloat16
-        if bits:
-            if c.bits != bits or c.group_size != 64:
-                return False
-            forms = ((torch.int32, a.head_dim * bits // 32), (bf, a.head_dim // 64), (bf, a.head_dim // 64))
-            parts = [(t, *f) for trip in (c.keys, c.values) for t, f in zip(trip, forms)]
-        else:
-            parts = [(t, bf, a.head_dim) for t in (c.keys, c.values)]
-        return all(t.device == self.h.device and t.dtype == dt and t.dim() == 4 and t.shape[2] >= need
-                   and t.shape == (1, a.num_key_value_heads, t.shape[2], width) and t.stride(3) == 1
-                   for t, dt, width in parts)
+    def _part_fits(self, t: torch.Tensor, dtype, width: int, need: int):
+        """(pointer, head stride, position stride) of a cache tensor if it is [1, KV heads, >= need, width]
+        of ``dtype`` on the engine's device with unit last stride, else None: the native step passes
+        pointers and strides, and the model's sizes for the rest."""
+        if t.dtype is not dtype or t.device != self._device:
+            return None
+        shape, stride = t.shape, t.stride()
+        if len(shape) != 4 or shape[0] != 1 or shape[1] != self.args.num_key_value_heads or shape[2] < need \
+                or shape[3] != width or stride[3] != 1:
+            return None
+        return t.data_ptr(), stride[1], stride[2]
 
     def _native_layers(self, M: int, cache: list, pos0: int) -> list[int] | None:
         """The layers of this step as ``dspark_verify_step`` takes them (the 8-byte fields of
@@ -346,40 +343,51 @@ class VerifyEngine:
         not one of the module's own in bf16 or a tensor is not what its kernel will take it for:
         those steps are enqueued launch by launch, with the checks (and refusals) of the single
         launches. Built from the modules and caches as they are now; nothing is kept."""
-        a = self.args
+        a, bf, need = self.args, torch.bfloat16, pos0 + M
         kv_bits = getattr(cache[0], "bits", 0)
         kind = QuantizedKVCache if kv_bits else KVCache
-        H = a.hidden_size
+        H, D = a.hidden_size, a.head_dim
+        W, G = D * kv_bits // 32, D // 64
         row = self.h.data_ptr()
         slot = {li: j for j, li in enumerate(self.tap)}
         fused, ld = self.fused.data_ptr(), self.fused.shape[1]
         pk, out = self._packed, []
+        norm, part = self._norm_fits, self._part_fits
         for li, (layer, c) in enumerate(zip(self.model.layers, cache)):
+            # the module's own tables, a quarter of an attribute's cost; what is not in them, by attribute
             at, mlp = layer.self_attn, layer.mlp
-            packs = [pk.get(id(mod)) for mod in (at.q_proj, at.k_proj, at.v_proj, at.o_proj)]
-            packs += [self._swiglu.get(id(mlp)), pk.get(id(mlp.down_proj))]
-            if None in packs or type(c) is not kind or not self._cache_fits(c, kv_bits, pos0 + M):
-                return None
-            if not (self._norm_fits(layer.input_layernorm, H) and self._norm_fits(layer.post_attention_layernorm, H)
-                    and self._norm_fits(at.q_norm, a.head_dim) and self._norm_fits(at.k_norm, a.head_dim)):
+            am, ab, lb = at._modules, at._buffers, layer._buffers
+            packs = [pk.get(id(am.get("q_proj"))), pk.get(id(am.get("k_proj"))), pk.get(id(am.get("v_proj"))),
+                     pk.get(id(am.get("o_proj"))), self._swiglu.get(id(mlp)), pk.get(id(mlp._modules.get("down_proj")))]
+            if None in packs or type(c) is not kind:
                 return None
             q, k, v, o, pair, down = packs
             if not q.bits == k.bits == v.bits or (q.n, k.n, v.n, o.n, pair.n, down.n) != self._widths \
                     or (q.k, k.k, v.k, pair.k, o.k, down.k) != (H, H, H, H, q.n, pair.n):
                 return None
-            out += [t.data_ptr() for t in (layer.input_layernorm, at.q_norm, at.k_norm, layer.post_attention_layernorm)]
+            n0, nq, nk, n1 = (lb.get("input_layernorm"), ab.get("q_norm"), ab.get("k_norm"),
+                              lb.get("post_attention_layernorm"))
+            if n0 is None or nq is None or nk is None or n1 is None:
+                n0, nq, nk, n1 = layer.input_layernorm, at.q_norm, at.k_norm, layer.post_attention_layernorm
+            if not (norm(n0, H) and norm(nq, D) and norm(nk, D) and norm(n1, H)):
+                return None
+            out += [n0.data_ptr(), nq.data_ptr(), nk.data_ptr(), n1.data_ptr()]
             out += [p.buf.data_ptr() for p in packs]
             out += [q.bits, o.bits, pair.bits, down.bits]
             if kv_bits:
-                (kw, ks, kb), (vw, vs, vb) = c.keys, c.values
-                if ks.stride() != kb.stride() or vs.stride() != vb.stride():
+                if c.bits != kv_bits or c.group_size != 64:
                     return None
-                out += [kw.data_ptr(), vw.data_ptr(), *kw.stride()[1:3], *vw.stride()[1:3]]
-                out += [t.data_ptr() for t in (ks, kb, vs, vb)]
-                out += [*ks.stride()[1:3], *vs.stride()[1:3]]
+                (kw, ks, kb), (vw, vs, vb) = c.keys, c.values
+                kw, vw = part(kw, torch.int32, W, need), part(vw, torch.int32, W, need)
+                ks, kb, vs, vb = part(ks, bf, G, need), part(kb, bf, G, need), part(vs, bf, G, need), part(vb, bf, G, need)
+                if None in (kw, ks, kb, vw, vs, vb) or ks[1:] != kb[1:] or vs[1:] != vb[1:]:
+                    return None
+                out += [kw[0], vw[0], *kw[1:], *vw[1:], ks[0], kb[0], vs[0], vb[0], *ks[1:], *vs[1:]]
             else:
-                kw, vw = c.keys, c.values
-                out += [kw.data_ptr(), vw.data_ptr(), *kw.stride()[1:3], *vw.stride()[1:3]] + [0] * 8
+                kw, vw = part(c.keys, bf, D, need), part(c.values, bf, D, need)
+                if kw is None or vw is None:
+                    return None
+                out += [kw[0], vw[0], *kw[1:], *vw[1:], 0, 0, 0, 0, 0, 0, 0, 0]
             j = slot.get(li)
             out += [row, H] if j is None else [fused + 2 * j * H, ld]
         return out
