@@ -481,18 +481,6 @@ struct MoeWorkspace {
   int gp_x, gp_h;
 };
 
-// Whether the buckets are large enough for the grouped prefill product (dspark_moe_wide.h), which
-// reads an expert's weights once for 32 or 64 rows, where the small-bucket kernels take 4 rows a pass
-// and 16 a workgroup. Its longer beginning and end cost small experts more. Measured, small-bucket /
-// grouped: 128 experts top 8, 2048 x 768, 4 bits: 3 rows a bucket 106 / 132 us, 4 rows 140 / 132, 32
-// rows 566 / 196; 8 bits: 3 rows 139 / 164, 4 rows 174 / 166; 32 experts top 4, 1024 x 384: 6 rows
-// 31.5 / 42.5, 8 rows 44.2 / 43.8, 16 rows 63 / 45.
-bool moe_wide(long M, long H, long I, long E, long k) {
-  const long rows = E * H * I >= 1L << 26 ? 4 : 8;
-  return M > 16 && M * k >= rows * E;
-}
-
-// (of both widths 4 bits need no less: their row tiles are no taller, so no fewer)
 MoeWorkspace moe_layout(long M, long H, long I, long E, long k, int bits) {
   MoeWorkspace w{};
   w.gu = moe_plan(H, I, E, M, true, bits);
@@ -510,7 +498,7 @@ MoeWorkspace moe_layout(long M, long H, long I, long E, long k, int bits) {
   w.part = o;    o += align256(sizeof(float) * (w.gu.part_floats > w.dn.part_floats ? w.gu.part_floats : w.dn.part_floats));
   w.gp_x = (int)((H / 64 + 31) / 32 * 32);
   w.gp_h = (int)((I / 64 + 31) / 32 * 32);
-  if (moe_wide(M, H, I, E, k)) {
+  if (moe_wide(M, H, I, E, k, bits)) {
     w.wide_mt = moe_wide_mt((long)P, E, bits);
     // sum over experts of ceil(rows / tile) <= P / tile + the experts that have rows
     w.max_tiles = (int)(P / (16 * w.wide_mt) + std::min((size_t)E, P));
@@ -694,7 +682,7 @@ extern "C" int dspark_gather_qmm(const void* x, int64_t ldx, int64_t K, const in
 
 extern "C" size_t dspark_moe_workspace(int64_t M, int64_t H, int64_t I, int64_t E, int64_t k) {
   if (check_route(M, E, k)) return 0;
-  return moe_layout(M, H, I, E, k, 4).total;
+  return std::max(moe_layout(M, H, I, E, k, 4).total, moe_layout(M, H, I, E, k, 8).total);  // of either width
 }
 
 namespace dspark {

@@ -6,6 +6,7 @@
 #include <mutex>
 
 #include "dspark_moe_cu.h"
+#include "dspark_moe_wide.h"
 
 namespace dspark {
 namespace {
@@ -73,7 +74,8 @@ using namespace dspark;
 extern "C" int dspark_moe_packed_plan(int64_t M, int64_t H, int64_t I, int64_t E, int64_t k, int bits,
                                      int32_t* out) {
   if (!out) return fail(DSPARK_ERR_ARG, "moe_packed_plan: null pointer");
-  out[0] = moe_cu_gate_up(M, H, I, E, k, bits) ? 1 : 0;
-  out[1] = 0;  // down: one workgroup per (expert, strip) (a per-CU down measured no faster)
+  const bool wide = moe_wide(M, H, I, E, k, bits);
+  out[0] = wide ? 2 : moe_cu_gate_up(M, H, I, E, k, bits) ? 1 : 0;
+  out[1] = wide ? 2 : 0;  // down: one workgroup per (expert, strip) (a per-CU down measured no faster)
   return DSPARK_OK;
 }

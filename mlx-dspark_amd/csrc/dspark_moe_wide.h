@@ -176,6 +176,8 @@ __global__ __launch_bounds__(kThreads, MT == 2 && BITS == 4 ? 3 : 2) void moe_wi
 
 }  // namespace wide
 
+// Whether the block runs its experts through this kernel rather than the small-bucket ones
+bool moe_wide(long M, long H, long I, long E, long k, int bits);
 // 16-row tiles of a workgroup for P pairs over E experts
 int moe_wide_mt(long P, long E, int bits);
 int launch_moe_wide(wide::MoeWideArgs a, bool swiglu, bool packed, int mt, int bits, hipStream_t s);

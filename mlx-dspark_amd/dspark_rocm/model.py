@@ -379,7 +379,8 @@ class VerifyEngine:
                     return None
                 (kw, ks, kb), (vw, vs, vb) = c.keys, c.values
                 kw, vw = part(kw, torch.int32, W, need), part(vw, torch.int32, W, need)
-                ks, kb, vs, vb = part(ks, bf, G, need), part(kb, bf, G, need), part(vs, bf, G, need), part(vb, bf, G, need)
+                ks, kb = part(ks, bf, G, need), part(kb, bf, G, need)
+                vs, vb = part(vs, bf, G, need), part(vb, bf, G, need)
                 if None in (kw, ks, kb, vw, vs, vb) or ks[1:] != kb[1:] or vs[1:] != vb[1:]:
                     return None
                 out += [kw[0], vw[0], *kw[1:], *vw[1:], ks[0], kb[0], vs[0], vb[0], *ks[1:], *vs[1:]]

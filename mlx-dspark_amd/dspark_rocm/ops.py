@@ -676,7 +676,7 @@ def moe_packable(experts: int, n: int, k: int, bits: int, group_size: int = GROU
     return int(_lib.load().dspark_moe_packed_bytes(experts, n, k, bits, group_size)) > 0
 
 
-MOE_KERNELS = ("expert x strip", "per CU")
+MOE_KERNELS = ("expert x strip", "per CU", "row tiles")
 
 
 def moe_packed_plan(M: int, H: int, I: int, E: int, k: int, bits: int) -> dict:

@@ -74,11 +74,31 @@ def test_prompt_chunks_match_float64(dev, bits, m, e, k, h, i):
         assert torch.equal(ops.moe_switch_glu(x, logits, *packed, k=k, bits=bits)[0], out)
 
 
-@pytest.mark.parametrize("m", [16, 17, 127, 128, 129])
-def test_both_sides_of_the_rule(dev, m):
-    """16 small experts, one each: eight rows a bucket from 128 tokens on."""
+def _row_tiles(m, e, k, h, i, bits):
+    """Whether the block of this shape runs the grouped prefill product."""
     from dspark_rocm import ops
 
+    plan = ops.moe_packed_plan(m, h, i, e, k, bits)
+    assert (plan["gate_up"] == "row tiles") == (plan["down"] == "row tiles")
+    return plan["gate_up"] == "row tiles"
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("m,e,k,h,i", [(512, 2, 1, 128, 128), (520, 8, 1, 256, 128), (301, 4, 2, 512, 384),
+                                       (1030, 1, 1, 640, 256), (345, 3, 3, 1024, 384), (515, 2, 2, 192, 64),
+                                       (65, 64, 8, 1024, 384), (97, 128, 8, 512, 256), (33, 16, 8, 2560, 640)])
+def test_row_tiles_match_float64(dev, bits, m, e, k, h, i):
+    """Sizes the rule sends to the grouped product, at the edges of its tiles, strips and chunks."""
+    assert _row_tiles(m, e, k, h, i, bits) or (h > 2048 and bits == 4)
+    test_prompt_chunks_match_float64(dev, bits, m, e, k, h, i)
+
+
+@pytest.mark.parametrize("m", [16, 17, 255, 256, 257])
+def test_both_sides_of_the_rule(dev, m):
+    """16 small experts, one each: from 256 tokens on."""
+    from dspark_rocm import ops
+
+    assert _row_tiles(m, 16, 1, 256, 192, 4) == (m >= 256)
     x, logits, mats = _block(dev, m, 16, 256, 192, 4, seed=m)
     out, inds, scores = ops.moe_switch_glu(x, logits, *mats, k=1, bits=4)
     _check(out, x, inds, scores, mats, 4, f"{m} rows")
@@ -89,6 +109,7 @@ def test_one_bucket_holds_every_token(dev, bits):
     """Every token on the same experts: their buckets take many row tiles, the others none."""
     from dspark_rocm import ops
 
+    assert _row_tiles(300, 32, 2, 256, 128, bits)
     x, logits, mats = _block(dev, 300, 32, 256, 128, bits)
     logits[:, 3] = 9.0
     logits[:, 30] = 8.0
@@ -104,13 +125,14 @@ def test_an_infinite_input_is_the_plain_product(dev, bits, packed):
     or a NaN, never a finite value), and the other rows keep their bits."""
     from dspark_rocm import ops
 
-    x, logits, mats = _block(dev, 64, 4, 256, 128, bits)
+    assert _row_tiles(320, 4, 1, 256, 128, bits)
+    x, logits, mats = _block(dev, 320, 4, 256, 128, bits)
     arg = [(ops.moe_pack(w, bits=bits), s, b) for w, s, b in mats] if packed else mats
     want, inds, scores = ops.moe_switch_glu(x, logits, *arg, k=1, bits=bits)
     x2 = x.clone()
     x2[5, 70] = float("inf")
     out = ops.moe_switch_glu(x2, logits, *arg, k=1, bits=bits)[0]
-    keep = torch.arange(64, device=dev) != 5
+    keep = torch.arange(320, device=dev) != 5
     assert torch.equal(out[keep], want[keep])
     e = int(inds[5, 0])
     gate, up, down = (_deq(*(a[e] for a in m), bits) for m in mats)
@@ -128,7 +150,8 @@ def test_infinite_rows_cost_no_more_than_their_terms(dev, bits, packed):
     product per output took 480), and no output is finite."""
     from dspark_rocm import ops
 
-    x, logits, mats = _block(dev, 200, 8, 1024, 512, bits)
+    assert _row_tiles(300, 8, 4, 1024, 512, bits)
+    x, logits, mats = _block(dev, 300, 8, 1024, 512, bits)
     arg = [(ops.moe_pack(w, bits=bits), s, b) for w, s, b in mats] if packed else mats
     x2 = x.clone()
     x2[:, 3] = float("inf")
