@@ -428,9 +428,9 @@ def verify_step_bytes(context: int, rows: int) -> tuple[int, int]:
 
 def bench_prefill_wide(dev, n: int = 12288, k: int = 4096, bits: int = 8, widths=(256, 512, 1024, 2048)) -> dict:
     """The prefill wide path on the 8B-shaped gate projection ([12288, 4096] 8-bit): per width M,
-    the stock path (torch dequantize + fp32 GEMM), the wide path (one dequantize launch + the same
-    fp32 GEMM, bit-identical) and its bf16 variant (dequantize to bf16 + bf16 GEMM), each called
-    eagerly back to back over 4 distinct matrices (as a prefill runs them); and the dequantize
+    the torch product (dequantize + fp32 GEMM), the wide path of bf16 rows (the matrix-core product
+    over the packed weight, which their stock path is too) and its bf16 variant (dequantize to bf16 +
+    bf16 GEMM), each called eagerly back to back over 4 distinct matrices (as a prefill runs them); and the dequantize
     kernel alone, graph-replayed (bytes: the packed weight, scales and biases read, the fp32
     weight written)."""
     import torch
@@ -445,7 +445,7 @@ def bench_prefill_wide(dev, n: int = 12288, k: int = 4096, bits: int = 8, widths
     for M in widths:
         x = torch.randn((M, k), generator=g, device=dev).to(torch.bfloat16)
         row = {"M": M}
-        for name, fn in (("stock_us", lambda m: wide_gemm._orig_call(m, x)),
+        for name, fn in (("stock_us", lambda m: m.torch_product(x)),
                          ("wide_us", lambda m: wide_gemm.wide_rows(m, x, exact=True)),
                          ("wide_bf16_us", lambda m: wide_gemm.wide_rows(m, x, exact=False))):
             ms = time_eager(lambda: [fn(m) for m in mats]) / len(mats)

@@ -46,13 +46,14 @@ inline long padded_groups(long K) { return (K / 64 + 31) / 32 * 32; }
 
 inline size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 
-Plan make_plan(long M, long K, long N, int bits) {
+Plan make_plan(long M, long K, long N) {
   Plan p{};
   const long G = K / 64;
   // The cheapest of the tile shapes and K slices under a model fitted to sweeps of them (M 20 to
   // 2048, N 512 to 17408, K 512 to 12288; cycles at the 2.07 GHz these kernels run at; the
   // picked plan is within 10% of the best one swept):
-  //   * a workgroup takes 350 + 100 nt + 45 mt nt cycles per group of K when two share a CU;
+  //   * a workgroup takes 350 + 100 nt + 45 mt nt cycles per group of K when two share a CU (of
+  //     either width: the cheaper loads of 4 bits go with the dearer unpacking);
   //   * two workgroups fill a CU, a CU's last one alone takes 1.4 of a share (2048 x 12288 x 4096:
   //     768 workgroups 247 us, but 777 rows of it in 432 workgroups 121 us, in 672 143 us);
   //   * K slices cost their fp32 partial sums, written and read once at 2000 bytes a cycle, and
@@ -122,7 +123,7 @@ using namespace dspark;
 
 extern "C" size_t dspark_qmm_wide_workspace(int64_t M, int64_t K, int64_t N, int bits, int group_size) {
   if (wide::check(M, K, N, bits, group_size)) return 0;
-  return wide::make_plan(M, K, N, bits).total;
+  return wide::make_plan(M, K, N).total;
 }
 
 extern "C" int dspark_qmm_wide(const void* x, int64_t ldx, int64_t M, int64_t K, const uint32_t* w, const void* scales,
@@ -134,7 +135,7 @@ extern "C" int dspark_qmm_wide(const void* x, int64_t ldx, int64_t M, int64_t K,
   if (ldx < K || ldx > (1L << 22) || ldy < N) return fail(DSPARK_ERR_SHAPE, "qmm_wide: ldx < K, ldx > 2^22 or ldy < N");
   if (!aligned(x, 16) || ldx % 8 || !aligned(w, 16) || !aligned(scales, 2) || !aligned(biases, 2))
     return fail(DSPARK_ERR_ALIGN, "qmm_wide: x and w must be 16-byte aligned, ldx %% 8 == 0");
-  const wide::Plan p = wide::make_plan(M, K, N, bits);
+  const wide::Plan p = wide::make_plan(M, K, N);
   if (!workspace || workspace_bytes < p.total)
     return fail(DSPARK_ERR_WORKSPACE, "qmm_wide: workspace %zu < %zu bytes", workspace_bytes, p.total);
   if (!aligned(workspace, 256)) return fail(DSPARK_ERR_ALIGN, "qmm_wide: workspace must be 256-byte aligned");
