@@ -430,9 +430,9 @@ def bench_prefill_wide(dev, n: int = 12288, k: int = 4096, bits: int = 8, widths
     """The prefill wide path on the 8B-shaped gate projection ([12288, 4096] 8-bit): per width M,
     the torch product (dequantize + fp32 GEMM), the wide path of bf16 rows (the matrix-core product
     over the packed weight, which their stock path is too) and its bf16 variant (dequantize to bf16 +
-    bf16 GEMM), each called eagerly back to back over 4 distinct matrices (as a prefill runs them); and the dequantize
-    kernel alone, graph-replayed (bytes: the packed weight, scales and biases read, the fp32
-    weight written)."""
+    bf16 GEMM), each called eagerly back to back over 4 distinct matrices (as a prefill runs them);
+    and the dequantize kernel alone, graph-replayed (bytes: the packed weight, scales and biases
+    read, the fp32 weight written)."""
     import torch
 
     from dspark_rocm import ops, wide_gemm

@@ -22,7 +22,7 @@
 // Measured (with the group sums and the K-slice sum): 2048 x 12288 x 4096, 8-bit, 241 us (857
 // TFLOP/s; a large bf16 matrix product of the library reaches 1150 to 1220 here) where an fp32
 // product of dequantized weights took 1450 us; 93 x 17408 x 5120, 4-bit, 43 us against 1363 us.
-// At 2048 rows the matrix pipe is busy 40% of the time and the VALU 50%: MFMAs in sequence with
+// At 2048 rows the matrix pipe is busy 38% of the time and the VALU issues 47% of it: MFMAs in sequence with
 // their FMAs, without the interleaving in tile_loop, took 280 us.
 #pragma once
 
