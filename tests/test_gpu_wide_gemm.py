@@ -6,7 +6,8 @@
   bf16 / fp16 outputs are that fp32 value rounded to the dtype;
 - the reference's load-bearing property (tests/test_wide_gemm.py:74-88): inside the scope the
   result is bit-identical to the stock path for fp32 / fp16 / bf16 activations at 4 and 8 bits,
-  over [1, L, K] leading dims, with a module bias; narrow calls fall through unchanged;
+  over [1, L, K] leading dims, with a module bias; narrow calls fall through unchanged. bf16 calls
+  run one kernel on both paths, so they are also held to the float64 product;
 - the verification accepts a shape where the paths agree and calibration never returns a
   threshold that does not verify (the divergence is simulated at the floor);
 - the exact=False variant (bf16 GEMM) within the qmm bar;
@@ -20,6 +21,7 @@ import pytest
 import torch
 
 from oracle import quant_ref
+from test_gpu_qmm_wide import _check as check_against_float64
 
 pytestmark = pytest.mark.gpu
 
@@ -86,6 +88,10 @@ def test_bit_identical_above_threshold(dev, bits, dtype):
             wg.wide_rows = real
     assert calls, "the forward did not take the wide path"
     assert got.shape == ref.shape and torch.equal(got, ref)
+    if lin.wide_kernel(x):
+        check_against_float64(got, x, lin.weight, lin.scales, lin.biases, bits)
+    else:
+        assert torch.equal(got, lin.torch_product(x))
 
 
 def test_leading_dims_bias_and_narrow_fall_through(dev):
@@ -136,16 +142,22 @@ def test_half_gemm_variant_within_the_qmm_bar(dev, bits):
     assert wg.verified_shapes([torch.nn.Sequential(lin)], 256, widths=(), exact=False) == [wg.shape_key(lin)]
 
 
-def test_prefill_fills_caches_identically_with_the_wide_path(dev, monkeypatch):
+@pytest.mark.parametrize("kernel", [True, False])
+def test_prefill_fills_caches_identically_with_the_wide_path(dev, monkeypatch, kernel):
     """prefill_plain (Target.prefill per chunk) with the wide path forced on (every shape verified at 256 rows) leaves
-    bit-identical caches and logits to the stock prefill, over two chunks (300 + 300 rows)."""
+    bit-identical caches and logits to the stock prefill, over two chunks (300 + 300 rows). Both with
+    the matrix-core kernel, which is then one call on both sides, and without it, where the wide path
+    is the dequantize kernel and the stock path the torch ops."""
     from _model_util import tiny_model
 
     from dspark_rocm import calibrate, wide_gemm
     from dspark_rocm.model import Target, prefill_plain
+    from dspark_rocm.nn import QuantizedLinear
 
     model = tiny_model(dev, seed=21, hidden_size=512, intermediate_size=1536)
     tgt = Target(model)
+    if not kernel:
+        monkeypatch.setattr(QuantizedLinear, "wide_kernel", lambda self, x: False)
     g = torch.Generator().manual_seed(6)
     ids = torch.randint(0, model.args.vocab_size, (1, 600), generator=g)
     monkeypatch.setattr(calibrate, "WIDE_GEMM_MIN_ROWS", None)
