@@ -68,13 +68,17 @@ __device__ __forceinline__ float moe_dequant_at(const MoeWideArgs& a, int e, int
 }
 
 // One output as the dequantized product in fp32, by a lane or (where its row has terms that are not
-// finite) the sum of those; for outputs whose factored sums are not finite
+// finite, and its weights are) the sum of those; for outputs whose factored sums are not finite
 template <int BITS, bool PW>
-__device__ __forceinline__ float moe_plain(const MoeWideArgs& a, int e, int which, const u16* xr, int n, bool take) {
+__device__ __forceinline__ float moe_plain(const MoeWideArgs& a, int e, int which, const u16* xr, int n, bool take,
+                                           bool whole) {
   auto weight = [&](int k) { return moe_dequant_at<BITS, PW>(a, e, which, n, k); };
   float acc;
-  if (!infinite_terms(xr, a.K, take, acc, weight) && take)
+  const bool terms = infinite_terms(xr, a.K, take, acc, weight);
+  if (take && (whole || !terms)) {
+    acc = 0.f;
     for (int k = 0; k < a.K && acc == acc; ++k) acc = __builtin_fmaf(bf2f(xr[k]), weight(k), acc);
+  }
   return acc;
 }
 
@@ -161,6 +165,10 @@ __global__ __launch_bounds__(kThreads, MT == 2 && BITS == 4 ? 3 : 2) void moe_wi
   if (!__builtin_amdgcn_ballot_w64(bad)) return;
   __threadfence_block();  // the wave's outputs are read back by other lanes
   const int n = n0 + wave * 16 * NW + lane;
+  bool whole[2];
+#pragma unroll
+  for (int j = 0; j < (SWIGLU ? 2 : 1); ++j)
+    whole[j] = infinite_weights(a.s[j], a.b[j], (long)tile.e * a.N + n - lane, min(16 * NW, a.N - n + lane), a.G, a.vec);
 #pragma unroll 1
   for (int m = 0; m < min(16 * MT, tile.rows); ++m) {
     u16* y = a.y + (long)(tile.p0 + m) * a.ldy + min(n, a.N - 1);
@@ -168,8 +176,8 @@ __global__ __launch_bounds__(kThreads, MT == 2 && BITS == 4 ? 3 : 2) void moe_wi
     if (!__builtin_amdgcn_ballot_w64(take)) continue;
     const u16* xr = a.x + (long)src(m) * a.ldx;
     float d[2];
-#pragma unroll 1
-    for (int j = 0; j < (SWIGLU ? 2 : 1); ++j) d[j] = moe_plain<BITS, PW>(a, tile.e, j, xr, n, take);
+#pragma unroll
+    for (int j = 0; j < (SWIGLU ? 2 : 1); ++j) d[j] = moe_plain<BITS, PW>(a, tile.e, j, xr, n, take, whole[j]);
     if (take) *y = h(d[0], d[SWIGLU ? 1 : 0]);
   }
 }

@@ -22,8 +22,8 @@
 // Measured (with the group sums and the K-slice sum): 2048 x 12288 x 4096, 8-bit, 241 us (857
 // TFLOP/s; a large bf16 matrix product of the library reaches 1150 to 1220 here) where an fp32
 // product of dequantized weights took 1450 us; 93 x 17408 x 5120, 4-bit, 43 us against 1363 us.
-// At 2048 rows the matrix pipe is busy 38% of the time and the VALU issues 47% of it: MFMAs in sequence with
-// their FMAs, without the interleaving in tile_loop, took 280 us.
+// At 2048 rows the matrix pipe is busy 38% of the time and the VALU issues 47% of it: MFMAs in sequence
+// with their FMAs, without the interleaving in tile_loop, took 280 us.
 #pragma once
 
 #include "dspark_qmm_core.h"
@@ -329,10 +329,11 @@ __device__ __forceinline__ float dequant_at(const Args& a, int n, int k) {
 
 // The factored sums turn an infinite x into a NaN (inf * 0 for a zero field, inf - inf with the bias
 // term) where the dequantized product is infinite, so outputs that are not finite are computed again.
-// Where the row of x has values that are not finite, their terms are the output: acc becomes the sum of
-// x[k] weight(k) over them, for the lanes of a wave (one output each, all of row xr) that take part.
-// False if the row has none. An infinity in one row of 93 x 17408 x 5120, 4-bit: 65 us, as without; in
-// every row 88; with each output's whole product by its lane 6.9 and 134 ms.
+// Where the row of x has values that are not finite (and the weights have none, infinite_weights), their
+// terms are the output: acc becomes the sum of x[k] weight(k) over them, for the lanes of a wave (one
+// output each, all of row xr) that take part. False if the row has none. An infinity in one row of 93 x
+// 17408 x 5120, 4-bit: 82 us where a call without takes 74; in every row 116; with each output's whole
+// product by its lane 6.9 and 134 ms.
 template <class W>
 __device__ __forceinline__ bool infinite_terms(const u16* xr, int K, bool take, float& acc, W weight) {
   const int lane = threadIdx.x & 63;
@@ -363,6 +364,29 @@ __device__ __forceinline__ bool infinite_terms(const u16* xr, int K, bool take, 
   return found;
 }
 
+// Whether a scale or bias of weight rows [n, n + rows) is not finite: by a wave, the rows' values in order
+__device__ __forceinline__ bool infinite_weights(const u16* s, const u16* b, long n, int rows, int G, bool vec) {
+  const long count = (long)rows * G;
+  s += n * G;
+  b += n * G;
+  bool any = false;
+  if (vec) {
+#pragma unroll 8
+    for (long i = 8 * (threadIdx.x & 63); i < count; i += 512) {
+      const u32x4_t x = ldg128(s + i), y = ldg128(b + i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        any |= (x[j] & 0x7F80u) == 0x7F80u || (x[j] & 0x7F800000u) == 0x7F800000u ||
+               (y[j] & 0x7F80u) == 0x7F80u || (y[j] & 0x7F800000u) == 0x7F800000u;
+    }
+  } else {
+#pragma unroll 8
+    for (long i = threadIdx.x & 63; i < count; i += 64)
+      any |= (s[i] & 0x7F80u) == 0x7F80u || (b[i] & 0x7F80u) == 0x7F80u;
+  }
+  return __builtin_amdgcn_ballot_w64(any) != 0;
+}
+
 // One output as the dequantized product in fp32
 template <int BITS>
 __device__ float plain_dot(const Args& a, int m, int n) {
@@ -379,12 +403,13 @@ __device__ __forceinline__ u16 finish(const Args& a, float v, int n) {
   return a.bias ? f2bf(bf2f(r) + bf2f(a.bias[n])) : r;  // the module's bias is added to the bf16 product
 }
 
-// Outputs y[m, n] again, by one wave: m is the wave's, n the lane's, take whether it has one.
+// Outputs y[m, n] again, by one wave: m is the wave's, n the lane's, take whether it has one, whole
+// whether weights of the wave's columns are not finite.
 template <int BITS>
-__device__ __forceinline__ void plain_outputs(const Args& a, int m, int n, bool take) {
+__device__ __forceinline__ void plain_outputs(const Args& a, int m, int n, bool take, bool whole) {
   float acc;
-  if (!infinite_terms(a.x + (long)m * a.ldx, a.K, take, acc, [&](int k) { return dequant_at<BITS>(a, n, k); }) && take)
-    acc = plain_dot<BITS>(a, m, n);
+  const bool terms = infinite_terms(a.x + (long)m * a.ldx, a.K, take, acc, [&](int k) { return dequant_at<BITS>(a, n, k); });
+  if (take && (whole || !terms)) acc = plain_dot<BITS>(a, m, n);
   if (take) a.y[(long)m * a.ldy + n] = finish(a, acc, n);
 }
 
@@ -463,10 +488,12 @@ __global__ __launch_bounds__(kThreads, 2) void wide_kernel(const Args a) {
   if (!__builtin_amdgcn_ballot_w64(bad)) return;
   __threadfence_block();  // the wave's outputs are read back by other lanes
   const int n = n0 + wave * 16 * NT + lane;
+  const int c0 = n0 + wave * 16 * NT;
+  const bool whole = infinite_weights(a.s, a.b, c0, min(16 * NT, a.N - c0), a.G, a.vec);
 #pragma unroll 1
   for (int m = m0; m < min(m0 + 16 * MT, a.M); ++m) {
     const bool take = lane < 16 * NT && n < a.N && not_finite(bf2f(a.y[(long)m * a.ldy + min(n, a.N - 1)]));
-    if (__builtin_amdgcn_ballot_w64(take)) plain_outputs<BITS>(a, m, n, take);
+    if (__builtin_amdgcn_ballot_w64(take)) plain_outputs<BITS>(a, m, n, take, whole);
   }
 }
 
@@ -496,6 +523,11 @@ __global__ __launch_bounds__(256) void wide_reduce_kernel(const Args a) {
     bad |= not_finite(v[j]) ? 1u << j : 0u;
   }
   if (!__builtin_amdgcn_ballot_w64(bad != 0)) return;
+  // the columns of the wave's 256 outputs, which may go on at the first one
+  const long i0 = i - 4 * (threadIdx.x & 63);
+  const int c0 = (int)(i0 % a.N), cols = min(256, a.N), to_end = min(cols, a.N - c0);
+  const bool whole = infinite_weights(a.s, a.b, c0, to_end, a.G, a.vec) ||
+                     infinite_weights(a.s, a.b, 0, cols - to_end, a.G, a.vec);
 #pragma unroll 1
   for (int j = 0; j < 4; ++j) {
     const int m = (int)((i + j) / a.N), n = (int)((i + j) - (long)m * a.N);
@@ -504,7 +536,7 @@ __global__ __launch_bounds__(256) void wide_reduce_kernel(const Args a) {
       const int row = __builtin_amdgcn_readlane(m, __builtin_ctzll(left));
       const bool take = ((bad >> j) & 1) && m == row;
       left &= ~__builtin_amdgcn_ballot_w64(take);
-      plain_outputs<BITS>(a, row, n, take);
+      plain_outputs<BITS>(a, row, n, take, whole);
     }
   }
 }

@@ -12,9 +12,9 @@ and :func:`wide_rows` makes the same call, so the bits agree. Such a shape is ve
 dequantized product at the qmm bar, and the crossover does not race the kernel against itself. For
 the other activation and scale dtypes the stock path dequantizes with torch elementwise ops --
 unpack through int64, convert, multiply, add: several passes over an ``N x K`` fp32 tensor -- and then
-runs one fp32 GEMM. The wide path produces the same fp32 weight in one pass (``dspark_qmm_dequantize``: ``(scale * q) + bias``, each operation rounded
-as torch rounds it, no fma contraction) and hands it to the same GEMM call with the same
-operands, so the bits agree by construction; :func:`verified_shapes` still checks every shape
+runs one fp32 GEMM. The wide path produces the same fp32 weight in one pass
+(``dspark_qmm_dequantize``: ``(scale * q) + bias``, each operation rounded as torch rounds it, no
+fma contraction) and hands it to the same GEMM call with the same operands, so the bits agree by construction; :func:`verified_shapes` still checks every shape
 before it is allowed, as the reference does (wide_gemm.py:263-306), so a change to either side
 turns a shape off instead of changing results. At prefill widths the win is the dequant chain
 (its time scales with ``N*K``, the GEMM's with ``M*N*K``), so it is largest at the narrow end

@@ -145,6 +145,26 @@ def test_an_infinite_input_is_the_plain_product(dev, bits, packed):
 
 @pytest.mark.parametrize("packed", [False, True])
 @pytest.mark.parametrize("bits", [4, 8])
+def test_an_infinite_weight_beside_an_infinite_row(dev, bits, packed):
+    """A gate of inf * 1 + 2 * -inf is a NaN, not an infinity, and so is the sum of its columns."""
+    from dspark_rocm import ops
+
+    x, logits, mats = _block(dev, 320, 4, 256, 128, bits)
+    inds = ops.moe_switch_glu(x, logits, *mats, k=1, bits=bits)[1]
+    e = int(inds[5, 0])
+    (_, gs, gb), (_, us, ub), (_, ds, db) = mats
+    gs[e, :, 0], gb[e, :, 0], gs[e, :, 1], gb[e, :, 1] = 0, 1, 0, -float("inf")
+    us[e], ub[e], ds[e], db[e] = 0, 0, 0, 1
+    ub[e, :, 2] = 1
+    x[:, 64:128], x[5, 3], x[5, 128:192] = 2 / 64, float("inf"), 1
+    arg = [(ops.moe_pack(w, bits=bits), s, b) for w, s, b in mats] if packed else mats
+    g = x[5].double() @ _deq(*(a[e] for a in mats[0]), bits)
+    assert bool(torch.isnan(g).all())
+    assert bool(torch.isnan(ops.moe_switch_glu(x, logits, *arg, k=1, bits=bits)[0][5]).all())
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("bits", [4, 8])
 def test_infinite_rows_cost_no_more_than_their_terms(dev, bits, packed):
     """An infinity in every row: the call stays within 20 times one without (about 3 measured; a whole
     product per output took 480), and no output is finite."""

@@ -133,6 +133,27 @@ def test_infinities_and_nans_follow_the_dequantized_product(dev, m, n, k, bits):
     assert torch.equal(torch.nan_to_num(got[odd], nan=7.0), torch.nan_to_num(want[odd], nan=7.0))
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("m,n,k", [(40, 200, 192), (96, 640, 2048)])
+def test_infinite_weights_beside_infinite_rows(dev, m, n, k, bits):
+    """A weight that is infinite too meets the row's finite values: an infinity of either sign, or a NaN."""
+    from dspark_rocm import ops, quant
+
+    w, s, b = _mats(dev, n, k, bits)
+    inf = float("inf")
+    b[8, 1], b[9, 1], s[130, 0] = -inf, inf, inf
+    s[8:10, 0], b[8:10, 0] = 0, 1
+    x = _x(dev, m, k)
+    x[2:8, 64:128] = x[2:8, 64:128].abs()
+    x[3, 5], x[7, 9], x[5, 70] = inf, -inf, inf
+    got = ops.quantized_matmul_wide(x, w, s, b, bits=bits).float()
+    want = (x.float() @ quant.dequantize(w, s, b, 64, bits).t()).to(torch.bfloat16).float()
+    odd = ~torch.isfinite(want)
+    assert bool(want[2, 8] == -inf) and bool(want[2, 9] == inf) and bool(want[3, 8].isnan())
+    assert torch.equal(~torch.isfinite(got), odd)
+    assert torch.equal(torch.nan_to_num(got[odd], nan=7.0), torch.nan_to_num(want[odd], nan=7.0))
+
+
 def test_capture_and_replay(dev):
     """A captured product replays on new inputs (its workspace is the graph's own)."""
     from dspark_rocm.nn import QuantizedLinear
