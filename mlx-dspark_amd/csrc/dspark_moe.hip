@@ -130,7 +130,8 @@ __device__ __forceinline__ void route_token(const RouteArgs& a, int t, int lane,
 }
 
 // Buckets the P = M k (token, slot) pairs of pair_e by expert; one workgroup of kRouteThreads.
-// counts [kRouteThreads] zeroed, pair_e written by any of its threads.
+// counts [kRouteThreads] zeroed, pair_e written by any of its threads. TILES: the buckets' row tiles too.
+template <bool TILES>
 __device__ __forceinline__ void bucket_pairs(const RouteArgs& a, int* pair_e, int* counts, u32* tmask) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, P = a.M * a.k;
   // ---- bucket the (token, slot) pairs by expert, stable in pair id. A token selects an
@@ -145,32 +146,38 @@ __device__ __forceinline__ void bucket_pairs(const RouteArgs& a, int* pair_e, in
   // exclusive scan of the bucket sizes by wave 0, 64 experts at a time; counts[e] becomes the
   // bucket start
   if (wave == 0) {
-    int carry = 0, tcarry = 0;
+    int carry = 0;
+    [[maybe_unused]] int tcarry = 0;
     for (int c0 = 0; c0 < a.E; c0 += 64) {
       const int e = c0 + lane;
       const int cnt = (e < a.E) ? counts[e] : 0;
-      const int nt = a.tiles ? (cnt + a.tile_rows - 1) / a.tile_rows : 0;
-      int incl = cnt, tincl = nt;
+      int incl = cnt;
 #pragma unroll
       for (int d = 1; d < 64; d <<= 1) {
-        const int o = __shfl_up(incl, d), to = __shfl_up(tincl, d);
-        if (lane >= d) {
-          incl += o;
-          tincl += to;
-        }
+        const int o = __shfl_up(incl, d);
+        if (lane >= d) incl += o;
       }
       if (e < a.E) {
         a.offsets[e] = carry + incl - cnt;
         counts[e] = carry + incl - cnt;
       }
-      for (int i = 0; i < nt; ++i)
-        a.tiles[tcarry + tincl - nt + i] = wide::MoeTile{e, carry + incl - cnt + i * a.tile_rows,
-                                                         min(a.tile_rows, cnt - i * a.tile_rows), 0};
+      if constexpr (TILES) {
+        const int nt = (cnt + a.tile_rows - 1) / a.tile_rows;
+        int tincl = nt;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+          const int o = __shfl_up(tincl, d);
+          if (lane >= d) tincl += o;
+        }
+        for (int i = 0; i < nt; ++i)
+          a.tiles[tcarry + tincl - nt + i] = wide::MoeTile{e, carry + incl - cnt + i * a.tile_rows,
+                                                           min(a.tile_rows, cnt - i * a.tile_rows), 0};
+        tcarry += __shfl(tincl, 63);
+      }
       carry += __shfl(incl, 63);
-      tcarry += __shfl(tincl, 63);
     }
     if (lane == 0) a.offsets[a.E] = carry;
-    if (a.tiles)
+    if constexpr (TILES)
       for (int i = tcarry + lane; i < a.max_tiles; i += 64) a.tiles[i] = wide::MoeTile{0, 0, 0, 0};
   }
   for (int t0 = 0; t0 < a.M; t0 += 64) {
@@ -201,7 +208,7 @@ __device__ __forceinline__ void bucket_pairs(const RouteArgs& a, int* pair_e, in
 constexpr size_t route_lds(size_t pairs) { return sizeof(int) * (pairs + 3 * kRouteThreads); }
 
 // One workgroup routes all M tokens (a wave per token, 16 at a time) and buckets the pairs.
-template <int NPL>
+template <int NPL, bool TILES>
 __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(const RouteArgs a) {
   extern __shared__ int lds[];
   int* counts = lds + a.M * a.k;
@@ -213,7 +220,7 @@ __global__ __launch_bounds__(kRouteThreads) void moe_route_kernel(const RouteArg
   // the grouped qmm's arrival counters (after the logits loads, which would otherwise wait
   // behind these stores)
   for (int i = threadIdx.x; i < a.nctr; i += kRouteThreads) a.ctr[i] = 0;
-  if (a.offsets) bucket_pairs(a, lds, counts, reinterpret_cast<u32*>(counts + kRouteThreads));
+  if (a.offsets) bucket_pairs<TILES>(a, lds, counts, reinterpret_cast<u32*>(counts + kRouteThreads));
 }
 
 // Many tokens: a wave per token over the whole chip, then one workgroup for the buckets.
@@ -223,13 +230,14 @@ __global__ __launch_bounds__(256) void moe_topk_kernel(const RouteArgs a) {
   if (t < a.M) route_token<NPL>(a, t, threadIdx.x & 63, nullptr);
 }
 
+template <bool TILES>
 __global__ __launch_bounds__(kRouteThreads) void moe_bucket_kernel(const RouteArgs a) {
   extern __shared__ int lds[];
   int* counts = lds + a.M * a.k;
   counts[threadIdx.x] = 0;
   for (int p = threadIdx.x; p < a.M * a.k; p += kRouteThreads) lds[p] = a.inds[p];
   for (int i = threadIdx.x; i < a.nctr; i += kRouteThreads) a.ctr[i] = 0;
-  bucket_pairs(a, lds, counts, reinterpret_cast<u32*>(counts + kRouteThreads));
+  bucket_pairs<TILES>(a, lds, counts, reinterpret_cast<u32*>(counts + kRouteThreads));
 }
 
 // ---------------------------------------------------------------- grouped expert qmm
@@ -405,11 +413,14 @@ template <int NPL>
 void launch_route_n(const RouteArgs& a, hipStream_t s) {
   const size_t lds = route_lds((size_t)a.M * a.k);
   if (a.M <= kRouteOneGroup) {
-    hipLaunchKernelGGL(moe_route_kernel<NPL>, dim3(1), dim3(kRouteThreads), lds, s, a);
+    if (a.tiles) hipLaunchKernelGGL((moe_route_kernel<NPL, true>), dim3(1), dim3(kRouteThreads), lds, s, a);
+    else hipLaunchKernelGGL((moe_route_kernel<NPL, false>), dim3(1), dim3(kRouteThreads), lds, s, a);
     return;
   }
   hipLaunchKernelGGL(moe_topk_kernel<NPL>, dim3((unsigned)((a.M + 3) / 4)), dim3(256), 0, s, a);
-  if (a.offsets) hipLaunchKernelGGL(moe_bucket_kernel, dim3(1), dim3(kRouteThreads), lds, s, a);
+  if (!a.offsets) return;
+  if (a.tiles) hipLaunchKernelGGL(moe_bucket_kernel<true>, dim3(1), dim3(kRouteThreads), lds, s, a);
+  else hipLaunchKernelGGL(moe_bucket_kernel<false>, dim3(1), dim3(kRouteThreads), lds, s, a);
 }
 
 int launch_route(const RouteArgs& a, hipStream_t s) {
